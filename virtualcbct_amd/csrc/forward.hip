@@ -20,22 +20,22 @@
 #include <vector>
 #include <cmath>
 
-#include "traverse.h"
+#include "runs.h"
 #include "vcbct_internal.h"
 
 namespace vcbct {
 
-// Occupancy of the ray kernels.  Their step loops wait on dependent LDS reads, scalar broadcasts and
-// gathers, and more resident waves hide that better than spilling a few registers costs: on the
-// 512x512x128 / 360-angle workload, k_forward takes 47.1 ms at its natural 75 VGPRs (6 waves per SIMD),
-// 45.0 ms held to 7 waves and 43.1 ms held to 8 (64 VGPRs, 56 bytes per lane spilled to scratch).  The
-// persistent batch kernel is fastest held to 7.  With the later step loop (76 VGPRs unbounded) the intensity
-// form takes 22.4 ms at 6 waves and 21.1 ms at both 7 and 8, while the log projection of the 256x256x64 /
-// 90-angle workload takes 1.58 ms at 7 (72 VGPRs, 28 bytes spilled) against 1.74 ms at 8: the projection
-// forms other than the intensity are held to 7.
+// Occupancy of the ray kernels.  The scatter walks step by step and waits on dependent LDS reads and scalar
+// broadcasts; more resident waves hide that better than spilling a few registers costs: held to 8 waves per SIMD.
+// The kernels that walk by runs (runs.h) keep eight gathers of a wave in flight instead, for which 5 waves per
+// SIMD have the registers: the 512x512x128 / 360-angle projection takes 10.7 ms at 5 waves, 10.9 at 6, 11.5 at 7
+// and 12.6 at 8 (where the scalar registers spill too); with the step walk it took 20.7 ms.  The ordered form needs
+// 4 (54.1 ms for the dual-energy gradient of a 512x512x64 / 360-angle problem; 54.6 at 5 with spills).
 #define VCBCT_WAVES8 __attribute__((amdgpu_waves_per_eu(8, 8)))
-#define VCBCT_WAVES7 __attribute__((amdgpu_waves_per_eu(7, 8)))
-#define VCBCT_WAVES_FWD(MODE) __attribute__((amdgpu_waves_per_eu((MODE) == VCBCT_MODE_INTENSITY ? 8 : 7, 8)))
+#define VCBCT_WAVES_RUN __attribute__((amdgpu_waves_per_eu(5, 5)))
+#define VCBCT_WAVES_ORDERED __attribute__((amdgpu_waves_per_eu(4, 4)))
+#define VCBCT_WAVES_COEF(MODE) \
+    __attribute__((amdgpu_waves_per_eu((MODE) == VCBCT_ADJ_LOSS ? 4 : 5, (MODE) == VCBCT_ADJ_LOSS ? 4 : 5)))
 
 // ------------------------------------------------------------------------------------------------
 // Volume re-layout.  Reference u16 [z][mat][y][x] -> device [y][x][z][8] (16-byte voxel, all materials;
@@ -314,6 +314,190 @@ struct AccumL<Ch4> {
     }
 };
 
+// The accumulators as the slice-run walk drives them (runs.h): gathers are raw buffer loads at a 32-bit byte offset,
+// so a slice outside the volume is a cell offset past the buffer's range (kOut: kOut cells are 2^31 bytes, and the
+// walk is taken for volumes of at most that) whose load returns zeros without touching memory.
+template <class VoxT>
+struct RunRec;  // a gathered record: what the sums need of a voxel
+template <>
+struct RunRec<float2> {
+    static constexpr int kShift = 3, kTerms = 2;
+    float v[2];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int off) {
+        typedef int I2 __attribute__((ext_vector_type(2)));
+        const I2 q = __builtin_amdgcn_raw_buffer_load_b64(b, off, 0, 0);
+        __builtin_memcpy(v, &q, sizeof v);
+    }
+    __device__ __forceinline__ float term(int m) const { return v[m]; }
+};
+template <>
+struct RunRec<Ch4> {
+    static constexpr int kShift = 4, kTerms = 4;
+    float v[4];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int off) {
+        typedef int I4 __attribute__((ext_vector_type(4)));
+        const I4 q = __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0);
+        __builtin_memcpy(v, &q, sizeof v);
+    }
+    __device__ __forceinline__ float term(int m) const { return v[m]; }
+};
+template <>
+struct RunRec<uint4> {
+    static constexpr int kShift = 4, kTerms = 6;
+    unsigned v[3];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int off) {
+        typedef int I3 __attribute__((ext_vector_type(3)));
+        const I3 q = __builtin_amdgcn_raw_buffer_load_b96(b, off, 0, 0);
+        v[0] = q.x;
+        v[1] = q.y;
+        v[2] = q.z;
+    }
+    __device__ __forceinline__ float term(int m) const { return (float)(m & 1 ? v[m >> 1] >> 16 : v[m >> 1] & 0xffffu); }
+};
+template <>
+struct RunRec<float4> {
+    static constexpr int kShift = 5, kTerms = 6;
+    float v[6];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t b, int off) {
+        typedef int I2 __attribute__((ext_vector_type(2)));
+        typedef int I4 __attribute__((ext_vector_type(4)));
+        const I4 q = __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0);
+        const I2 w = __builtin_amdgcn_raw_buffer_load_b64(b, off + 16, 0, 0);
+        __builtin_memcpy(v, &q, sizeof q);
+        __builtin_memcpy(v + 4, &w, sizeof w);
+    }
+    __device__ __forceinline__ float term(int m) const { return v[m]; }
+};
+
+template <class VoxT>
+struct RunAcc {
+    typedef RunRec<VoxT> Q;
+    static constexpr int kOut = (int)(0x80000000u >> Q::kShift);
+        // gathers in flight per wave (512x512x128 / 360 angles: 10.6 ms with 8, 10.6 with 4; 320x320x77 / 120 angles: 2.12
+    // against 2.25 ms); the two-load FP32 record half of that
+    static constexpr int kBatch = sizeof(Q) <= 16 ? 8 : 4;
+    __amdgpu_buffer_rsrc_t buf;
+    float L[VCBCT_MAX_MAT];
+    __device__ __forceinline__ RunAcc(const VoxT* vox, const ProjGeom& g) {
+        const unsigned bytes = (unsigned)((size_t)g.N * g.N * g.Nz << Q::kShift);
+        buf = __builtin_amdgcn_make_buffer_rsrc((void*)vox, (short)0, (int)bytes, 0x00020000);
+#pragma unroll
+        for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = 0.0f;
+    }
+    __device__ __forceinline__ void load(int cell, Q& q) const { q.load(buf, (int)((unsigned)cell << Q::kShift)); }
+    __device__ __forceinline__ void add(const Q& q, float len) {
+#pragma clang fp contract(fast)
+#pragma unroll
+        for (int m = 0; m < Q::kTerms; ++m) L[m] += q.term(m) * len;
+    }
+    // pieces [pa, pb) of the list: before first_new to offset zo, the rest to zn; the lane's length of piece px is lo
+    __device__ __forceinline__ void run(const PieceRec* p, int pa, int pb, int px, int first_new, float lo, int zo,
+                                        int zn, float K) {
+        int i = pa;
+        for (; i + kBatch <= pb; i += kBatch) {
+            PieceRec t[kBatch];
+            Q q[kBatch];
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b) t[b] = p[i + b];
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b) load(t[b].cb + (i + b < first_new ? zo : zn), q[b]);
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b) add(q[b], i + b == px ? lo : t[b].len * K);
+        }
+        if (i < pb) {  // the rest as one batch: past the end, the last piece again with length 0
+            PieceRec t[kBatch - 1];
+            Q q[kBatch - 1];
+#pragma unroll
+            for (int b = 0; b < kBatch - 1; ++b) t[b] = p[i + b < pb ? i + b : pb - 1];
+#pragma unroll
+            for (int b = 0; b < kBatch - 1; ++b)
+                load(t[b].cb + ((i + b < pb ? i + b : pb - 1) < first_new ? zo : zn), q[b]);
+#pragma unroll
+            for (int b = 0; b < kBatch - 1; ++b) add(q[b], i + b >= pb ? 0.0f : i + b == px ? lo : t[b].len * K);
+        }
+    }
+};
+
+// The ordered walk's sums: a piece's length as (float)(len K), the factors applied term by term.  The step walk adds a
+// step's first gather after its second, except over the FP32 maps (AccumL).
+template <class VoxT>
+struct OrderedAcc : RunAcc<VoxT> {
+    typedef RunRec<VoxT> Q;
+    using RunAcc<VoxT>::kBatch;
+    static constexpr bool kSecondFirst = !std::is_same<VoxT, float4>::value;
+    __device__ __forceinline__ OrderedAcc(const VoxT* vox, const ProjGeom& g) : RunAcc<VoxT>(vox, g) {}
+    __device__ __forceinline__ void run_ordered(const OrderedPiece* p, int pa, int pb, int px, int first_new, float lo,
+                                                int zo, int zn, double K) {
+        for (int i = pa; i < pb; i += kBatch) {
+            OrderedPiece t[kBatch];
+            Q q[kBatch];
+            // (past the end: the last piece again, with length 0 off the volume)
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b) t[b] = p[i + b < pb ? i + b : pb - 1];
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b) {
+                const int k = i + b < pb ? i + b : pb - 1;
+                this->load(t[b].cb + (k < first_new || k == px ? zo : zn), q[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b)
+                this->add(q[b], i + b >= pb ? 0.0f : i + b == px ? lo : (float)(t[b].len * K));
+        }
+    }
+};
+
+// The line integrals of one wave's rays into L: by runs where the wave's lanes share their xy path, no lane can meet
+// two slice planes in one step and the volume is within the gathers' reach, else step by step.  ORDERED: bit for bit
+// the step walk's sums (plane grids off the voxel grid keep that walk).  Returns the lane's cos^3 factor.
+template <bool ORDERED, class VoxT>
+__device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double sn, double xc, double yc, int j, int jj,
+                                           bool active, const VoxT* __restrict__ vox, float (&L)[VCBCT_MAX_MAT],
+                                           WalkLds* lds) {
+    RayCtx r;
+    ray_setup(g, c, sn, xc, yc, active ? j : 0, jj, r);
+    share_xy_path(r);
+    int klo, khi;
+    z_step_range(g, r, active, klo, khi);
+    const int kmin = wave_min(klo);
+    const int kmax = wave_max(khi);
+#pragma unroll
+    for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = 0.0f;
+    if (kmin > kmax) return r.leng;  // no lane reaches the volume's z band
+    const bool same = __all((int)r.swap == __builtin_amdgcn_readfirstlane((int)r.swap));
+    // (the ordered walk hands pieces over when any lane crosses a slice, in range or not)
+    float slope = (ORDERED ? active && r.hit : klo <= khi) ? run_slope(r) : 0.0f;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) slope = fmaxf(slope, __shfl_xor(slope, o, 64));
+    int nb = same && (size_t)g.N * g.N * g.Nz <= (size_t)RunAcc<VoxT>::kOut ? run_block_steps(g, slope) : 0;
+    nb = __builtin_amdgcn_readfirstlane(nb);
+    if (ORDERED && !g.aligned) nb = 0;
+    if (nb > 0) {
+        if constexpr (ORDERED) {
+            OrderedAcc<VoxT> acc(vox, g);
+            walk_runs_ordered(g, r, active, kmin, kmax, nb, acc, &lds->ordered);
+#pragma unroll
+            for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
+        } else {
+            RunAcc<VoxT> acc(vox, g);
+            if (g.aligned) walk_runs<true>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
+            else walk_runs<false>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
+#pragma unroll
+            for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
+        }
+    } else {
+        AccumL<VoxT> acc;
+        acc.vox = vox;
+        acc.Nz = g.Nz;
+#pragma unroll
+        for (int m = 0; m < VCBCT_MAX_MAT; ++m) acc.L[m] = 0.0f;
+        traverse_lane(g, r, active, kmin, kmax, acc, ORDERED && same ? &lds->table : nullptr);
+        acc.finish();
+#pragma unroll
+        for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
+    }
+    return r.leng;
+}
+
 // The channel volume of a material volume, one thread per voxel: c_k = sum_m b[m][k] rho_m in FP32, m
 // ascending (with the identity mix c_k = rho_k exactly).  SrcT uint4: one u16 record per voxel; float4: two
 // FP32 records per voxel.  DstT float2 or Ch4 (channels past mix.nch are zero).
@@ -375,7 +559,7 @@ __device__ __forceinline__ double spectral_x(const float (&L)[VCBCT_MAX_MAT], in
     double x = 0.0;
 #pragma unroll
     for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-        if (m < nmat) x += ldg(mu, m * NE + e) * (double)L[m];
+        if (m < nmat) x += ldk(mu, m * NE + e) * (double)L[m];
     return x * inv_xf;
 }
 
@@ -386,7 +570,7 @@ __device__ __forceinline__ double spectral_xmin(const float (&L)[VCBCT_MAX_MAT],
     double xmin = 0.0;
     bool first = true;
     for (int e = 0; e < NE; ++e) {
-        if (!(ldg(pdf, e) > 0.0)) continue;
+        if (!(ldk(pdf, e) > 0.0)) continue;
         const double x = spectral_x(L, nmat, mu, NE, e, inv_xf);
         if (first || x < xmin) xmin = x;
         first = false;
@@ -403,12 +587,12 @@ __device__ __forceinline__ double spectral_shifted(const float (&L)[VCBCT_MAX_MA
                                                    const double* __restrict__ ch = nullptr, int nch = 0) {
     double se = 0.0;
     for (int e = 0; e < NE; ++e) {
-        const double we = ldg(pdf, e) * exp(-(spectral_x(L, nmat, mu, NE, e, inv_xf) - xmin));
+        const double we = ldk(pdf, e) * exp(-(spectral_x(L, nmat, mu, NE, e, inv_xf) - xmin));
         se += we;
         if (MUB) {
 #pragma unroll
             for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                if (m < nch) mub[m] += we * ldg(ch, m * NE + e);
+                if (m < nch) mub[m] += we * ldk(ch, m * NE + e);
         }
     }
     return se;
@@ -420,7 +604,7 @@ __device__ __forceinline__ float intensity_exact(const float (&L)[VCBCT_MAX_MAT]
                                                  const double* __restrict__ mu, const double* __restrict__ pdf, int NE,
                                                  double inv_xf, double leng) {
     float s = 0.0f;
-    for (int e = 0; e < NE; ++e) s += (float)(ldg(pdf, e) * exp(-spectral_x(L, nmat, mu, NE, e, inv_xf)) * leng);
+    for (int e = 0; e < NE; ++e) s += (float)(ldk(pdf, e) * exp(-spectral_x(L, nmat, mu, NE, e, inv_xf)) * leng);
     return s;
 }
 
@@ -445,6 +629,13 @@ __device__ __forceinline__ double mubar_opaque(const float (&L)[VCBCT_MAX_MAT], 
 #pragma unroll
     for (int m = 0; m < VCBCT_MAX_MAT; ++m) mub[m] /= se;
     return xmin - log(se / sw);
+}
+
+__device__ __forceinline__ bool all_zero(const float (&L)[VCBCT_MAX_MAT]) {
+    bool z = true;
+#pragma unroll
+    for (int m = 0; m < VCBCT_MAX_MAT; ++m) z = z && L[m] == 0.0f;
+    return z;
 }
 
 // Counts the charged segments of a ray (the algorithmic work unit of the roofline model).
@@ -519,42 +710,37 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
                                              const double* __restrict__ pdf, const float* __restrict__ muf,
                                              const float* __restrict__ pdff, int NE, double inv_xf, int nl, int a,
                                              int rg, int jj, float* __restrict__ out, float* __restrict__ aux,
-                                             WaveLds* steps) {
+                                             WalkLds* steps) {
     const int lane = threadIdx.x & 63;
     const int j = rg * 64 + lane;
     const bool active = j < g.H;
 
-    const double c = ldg(tab, a), sn = ldg(tab, g.nAng + a), xc = ldg(tab, 2 * g.nAng + a),
-                 yc = ldg(tab, 3 * g.nAng + a);
+    const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
+                 yc = ldk(tab, 3 * g.nAng + a);
     const size_t o = (size_t)a * g.H * g.W + (size_t)(g.H - 1 - j) * g.W + jj;
     if (MODE == VCBCT_MODE_SEGCOUNT) {
         CountSeg cnt;
-        traverse_wave(g, c, sn, xc, yc, j, jj, active, cnt, steps);
+        traverse_wave(g, c, sn, xc, yc, j, jj, active, cnt, &steps->table);
         if (active) stg(aux, o, (float)cnt.n);
         return;
     }
-    AccumL<VoxT> acc;
-    acc.vox = vox;
-    acc.Nz = g.Nz;
-#pragma unroll
-    for (int m = 0; m < VCBCT_MAX_MAT; ++m) acc.L[m] = 0.0f;
-    const double leng = traverse_wave(g, c, sn, xc, yc, j, jj, active, acc, steps);
-    acc.finish();
+    float L[VCBCT_MAX_MAT];
+    const double leng = sum_wave<false>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
     if (!active) return;
 
     if (MODE == VCBCT_MODE_LINEINT) {
-        for (int m = 0; m < g.nmat; ++m) stg(aux, o * g.nmat + m, (float)acc.L[m]);
+        for (int m = 0; m < g.nmat; ++m) stg(aux, o * g.nmat + m, (float)L[m]);
         return;
     }
     if (MODE == VCBCT_MODE_LOGPROJ && aux) {  // the nl line integrals, kept for the backward pass ([term][ray])
         const size_t nrays = (size_t)g.nAng * g.H * g.W;
 #pragma unroll
         for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-            if (m < nl) stg(aux, (size_t)m * nrays + o, acc.L[m]);
+            if (m < nl) stg(aux, (size_t)m * nrays + o, L[m]);
     }
     bool zero = true;
 #pragma unroll
-    for (int m = 0; m < VCBCT_MAX_MAT; ++m) zero = zero && (acc.L[m] == 0.0);
+    for (int m = 0; m < VCBCT_MAX_MAT; ++m) zero = zero && (L[m] == 0.0);
     if (MODE == VCBCT_MODE_INTENSITY) {
         // sum_e pdf_e * exp(-transp_e / xf) * leng, accumulated in FP32 in e order (P/reprojectionOnGPU.cu:432,
         // 1038-1044).  A ray that charges nothing sums the reference's own terms, float(pdf_e * 1.0 * leng), bit
@@ -563,42 +749,50 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
         // below the FP32 accumulation of the line integrals.  exp(-x) = 2^(-x log2 e).
         float s = 0.0f;
         if (zero) {
-            for (int e = 0; e < NE; ++e) s += (float)(ldg(pdf, e) * 1.0 * leng);
+            for (int e = 0; e < NE; ++e) s += (float)(ldk(pdf, e) * 1.0 * leng);
         } else {
             const float lf = (float)leng;
             const float k2 = (float)(-inv_xf * 1.4426950408889634);
+#pragma unroll 4
             for (int e = 0; e < NE; ++e) {
                 float tr = 0.0f;
 #pragma unroll
                 for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nl) tr = fmaf(ldg(muf, m * NE + e), acc.L[m], tr);
-                s += ldg(pdff, e) * exp2f(tr * k2) * lf;
+                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
+                s += ldk(pdff, e) * exp2f(tr * k2) * lf;
             }
             // opaque ray: the FP32 exponentials underflow; the reference's own FP64 terms instead
-            if (s < 1e-30f) s = intensity_exact(acc.L, nl, mu, pdf, NE, inv_xf, leng);
+            if (s < 1e-30f) s = intensity_exact(L, nl, mu, pdf, NE, inv_xf, leng);
         }
         stg(out, o, s);
     } else {  // VCBCT_MODE_LOGPROJ: p = -log(sum_e pdf_e e^{-mu.L/xf} / sum_e pdf_e); FP32 terms, FP64 sums
         double sw = 0.0, se = 0.0;
         const float k2 = (float)(-inv_xf * 1.4426950408889634);
-        for (int e = 0; e < NE; ++e) {
-            float tr = 0.0f;
+        if (!__any(!zero)) {  // rays that charge nothing: every exponential is 1
+#pragma unroll 4
+            for (int e = 0; e < NE; ++e) sw += ldk(pdf, e);
+            se = sw;
+        } else {
+#pragma unroll 4
+            for (int e = 0; e < NE; ++e) {
+                float tr = 0.0f;
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                if (m < nl) tr = fmaf(ldg(muf, m * NE + e), acc.L[m], tr);
-            const double pe = ldg(pdf, e);
-            sw += pe;
-            se += pe * (double)exp2f(tr * k2);
+                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
+                const double pe = ldk(pdf, e);
+                sw += pe;
+                se += pe * (double)exp2f(tr * k2);
+            }
         }
         // opaque ray (the FP32 exponentials underflow): FP64 terms relative to the smallest exponent
-        const double p = se < 1e-30 * sw ? logproj_opaque(acc.L, nl, mu, pdf, NE, inv_xf, sw) : -log(se / sw);
+        const double p = se < 1e-30 * sw ? logproj_opaque(L, nl, mu, pdf, NE, inv_xf, sw) : -log(se / sw);
         stg(out, o, (float)p);
     }
 }
 
 // WPB waves per block (TileShape: rgb * cols); the block's waves share nothing but the LDS allocation.
 template <int MODE, class VoxT, int WPB>
-__global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_FWD(MODE) void k_forward(ProjGeom g, const double* __restrict__ tab,
+__global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_RUN void k_forward(ProjGeom g, const double* __restrict__ tab,
                                                                  const VoxT* __restrict__ vox,
                                                                  const double* __restrict__ mu,
                                                                  const double* __restrict__ pdf,
@@ -606,7 +800,7 @@ __global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_FWD(MODE) void k_forward(Proj
                                                                  const float* __restrict__ pdff, int NE,
                                                                  double inv_xf, int nl, int a0, int nA, TileMap tm,
                                                                  float* __restrict__ out, float* __restrict__ aux) {
-    __shared__ WaveLds steps[WPB];
+    __shared__ WalkLds steps[WPB];
     const Tile t = tile_map(tm, nA);
     if (t.col >= g.W || t.a >= nA || t.rg * 64 >= g.H) return;  // wave out of range: uniform exit
     forward_wave<MODE, VoxT>(g, tab, vox, mu, pdf, muf, pdff, NE, inv_xf, nl, a0 + t.a, t.rg, t.col, out, aux,
@@ -631,9 +825,9 @@ __device__ __forceinline__ int find_problem(const BatchProblem* __restrict__ pr,
 }
 
 template <class VoxT>
-__global__ __launch_bounds__(256) VCBCT_WAVES7 void k_forward_batch(const BatchProblem* __restrict__ pr, int np,
+__global__ __launch_bounds__(256) VCBCT_WAVES_RUN void k_forward_batch(const BatchProblem* __restrict__ pr, int np,
                                                        const int* __restrict__ xcd_total, int* __restrict__ counters) {
-    __shared__ WaveLds steps[4];
+    __shared__ WalkLds steps[4];
     const int home = blockIdx.x & 7;
     const int lane = threadIdx.x & 63;
     for (int qi = 0; qi < 8; ++qi) {
@@ -666,8 +860,8 @@ __global__ __launch_bounds__(256) VCBCT_WAVES7 void k_forward_batch(const BatchP
 // own blocks with its tile map (each problem's block count is a multiple of 8, so block b still runs on XCD
 // b % 8 and the map's XCD assignment carries over).
 template <class VoxT>
-__global__ __launch_bounds__(256) VCBCT_WAVES8 void k_forward_flat(const BatchProblem* __restrict__ pr, int np) {
-    __shared__ WaveLds steps[4];
+__global__ __launch_bounds__(256) VCBCT_WAVES_RUN void k_forward_flat(const BatchProblem* __restrict__ pr, int np) {
+    __shared__ WalkLds steps[4];
     const int b = blockIdx.x;
     int lo = 0, hi = np - 1;
     while (lo < hi) {  // last problem whose first block <= b
@@ -780,14 +974,14 @@ struct ScatterG {
 // VoxT float4: the FP32 maps (mu / muf the material tables, nl = nmat); float2 / Ch4: their channel volume
 // (mu / muf the channel tables, nl = nch).
 template <int MODE, class VoxT>
-__global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_coef(ProjGeom g, const double* __restrict__ tab,
+__global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(ProjGeom g, const double* __restrict__ tab,
                                                       const VoxT* __restrict__ vox, const double* __restrict__ mu,
                                                       const double* __restrict__ pdf, const float* __restrict__ muf,
                                                       const double* __restrict__ ch, int nch, int NE, double inv_xf,
                                                       int nl, TileMap tm, const float* __restrict__ tg,
                                                       float* __restrict__ coef, double* __restrict__ loss) {
-    __shared__ WaveLds step_tabs[4];
-    WaveLds* steps = &step_tabs[threadIdx.x >> 6];
+    __shared__ WalkLds step_tabs[4];
+    WalkLds* steps = &step_tabs[threadIdx.x >> 6];
     const Tile t = tile_map(tm, g.nAng);
     const int lane = threadIdx.x & 63;
     const int j = t.rg * 64 + lane;
@@ -795,39 +989,47 @@ __global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_coef(ProjGeom g, c
     const int a = t.a;
     if (jj >= g.W || a >= g.nAng || t.rg * 64 >= g.H) return;  // wave out of range: uniform exit
     const bool active = j < g.H;
-    const double c = ldg(tab, a), sn = ldg(tab, g.nAng + a), xc = ldg(tab, 2 * g.nAng + a),
-                 yc = ldg(tab, 3 * g.nAng + a);
-    AccumL<VoxT> acc;
-    acc.vox = vox;
-    acc.Nz = g.Nz;
-#pragma unroll
-    for (int m = 0; m < VCBCT_MAX_MAT; ++m) acc.L[m] = 0.0f;
-    traverse_wave(g, c, sn, xc, yc, j, jj, active, acc, steps);
-    acc.finish();  // (the pipelined accumulators add their last gather here)
+    const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
+                 yc = ldk(tab, 3 * g.nAng + a);
+    float L[VCBCT_MAX_MAT];
+    sum_wave<MODE == VCBCT_ADJ_LOSS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
 
     double lossc = 0.0;
     if (active) {
         // the exponent and its exponential in FP32 (relative error ~1e-6 per term), the sums in FP64
         double sw = 0.0, se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
         const float k2 = (float)(-inv_xf * 1.4426950408889634);
-        for (int e = 0; e < NE; ++e) {
-            float tr = 0.0f;
+        if (__any(!all_zero(L))) {
+#pragma unroll 4
+            for (int e = 0; e < NE; ++e) {
+                float tr = 0.0f;
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                if (m < nl) tr = fmaf(ldg(muf, m * NE + e), acc.L[m], tr);
-            const double pe = ldg(pdf, e);
-            const double we = pe * (double)exp2f(tr * k2);
-            sw += pe;
-            se += we;
+                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
+                const double pe = ldk(pdf, e);
+                const double we = pe * (double)exp2f(tr * k2);
+                sw += pe;
+                se += we;
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                if (m < nch) mub[m] += we * ldg(ch, m * NE + e);
+                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    if (m < nch) mub[m] += we * ldk(ch, m * NE + e);
+            }
+        } else {  // rays that charge nothing: every exponential is 1
+#pragma unroll 4
+            for (int e = 0; e < NE; ++e) {
+                const double pe = ldk(pdf, e);
+                sw += pe;
+#pragma unroll
+                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    if (m < nch) mub[m] += pe * ldk(ch, m * NE + e);
+            }
+            se = sw;
         }
         const size_t nrays = (size_t)g.nAng * g.H * g.W;
         const size_t o = (size_t)a * g.H * g.W + (size_t)(g.H - 1 - j) * g.W + jj;
         double p;
         if (se < 1e-30 * sw) {  // opaque ray: FP64 terms relative to the smallest exponent
-            p = mubar_opaque(acc.L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, nch);
+            p = mubar_opaque(L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, nch);
         } else {
             p = -log(se / sw);
 #pragma unroll
@@ -861,14 +1063,14 @@ __global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_coef(ProjGeom g, c
 // NCH: the channel count (the arrays of the spectral loop stay in registers).  VoxT float4: the FP32 maps (the
 // exponents over the material tables); float2 / Ch4: the joint basis's channel volume (over the channel tables).
 template <int NCH, class VoxT>
-__global__ __launch_bounds__(256) VCBCT_WAVES7 void k_adjoint_coef_multi(ProjGeom g, const double* __restrict__ tab,
+__global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(ProjGeom g, const double* __restrict__ tab,
                                                                          const VoxT* __restrict__ vox, SpecSet ss,
                                                                          double inv_xf, TileMap tm,
                                                                          const float* __restrict__ tg,
                                                                          float* __restrict__ coef,
                                                                          double* __restrict__ loss) {
-    __shared__ WaveLds step_tabs[4];
-    WaveLds* steps = &step_tabs[threadIdx.x >> 6];
+    __shared__ WalkLds step_tabs[4];
+    WalkLds* steps = &step_tabs[threadIdx.x >> 6];
     const Tile t = tile_map(tm, g.nAng);
     const int lane = threadIdx.x & 63;
     const int j = t.rg * 64 + lane;
@@ -876,15 +1078,10 @@ __global__ __launch_bounds__(256) VCBCT_WAVES7 void k_adjoint_coef_multi(ProjGeo
     const int a = t.a;
     if (jj >= g.W || a >= g.nAng || t.rg * 64 >= g.H) return;  // wave out of range: uniform exit
     const bool active = j < g.H;
-    const double c = ldg(tab, a), sn = ldg(tab, g.nAng + a), xc = ldg(tab, 2 * g.nAng + a),
-                 yc = ldg(tab, 3 * g.nAng + a);
-    AccumL<VoxT> acc;
-    acc.vox = vox;
-    acc.Nz = g.Nz;
-#pragma unroll
-    for (int m = 0; m < VCBCT_MAX_MAT; ++m) acc.L[m] = 0.0f;
-    traverse_wave(g, c, sn, xc, yc, j, jj, active, acc, steps);
-    acc.finish();  // (the pipelined accumulators add their last gather here)
+    const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
+                 yc = ldk(tab, 3 * g.nAng + a);
+    float L[VCBCT_MAX_MAT];
+    sum_wave<true>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
 
     double lossc = 0.0;
     if (active) {
@@ -894,6 +1091,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES7 void k_adjoint_coef_multi(ProjGeo
         double cacc[NCH];
 #pragma unroll
         for (int m = 0; m < NCH; ++m) cacc[m] = 0.0;
+        const bool charges = __any(!all_zero(L));  // (wave-uniform)
         for (int s = 0; s < ss.nspec; ++s) {
             const int NE = ss.NE[s];
             constexpr bool CHV = !std::is_same<VoxT, float4>::value;  // channel volume
@@ -903,21 +1101,33 @@ __global__ __launch_bounds__(256) VCBCT_WAVES7 void k_adjoint_coef_multi(ProjGeo
             const float* __restrict__ muf = CHV ? ss.chf[s] : ss.muf[s];
             const double* __restrict__ ch = ss.ch[s];
             double sw = 0.0, se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
-            for (int e = 0; e < NE; ++e) {
-                float tr = 0.0f;
+            if (charges) {
+#pragma unroll 4
+                for (int e = 0; e < NE; ++e) {
+                    float tr = 0.0f;
 #pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nl) tr = fmaf(ldg(muf, m * NE + e), acc.L[m], tr);
-                const double pe = ldg(pdf, e);
-                const double we = pe * (double)exp2f(tr * k2);
-                sw += pe;
-                se += we;
+                    for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                        if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
+                    const double pe = ldk(pdf, e);
+                    const double we = pe * (double)exp2f(tr * k2);
+                    sw += pe;
+                    se += we;
 #pragma unroll
-                for (int m = 0; m < NCH; ++m) mub[m] += we * ldg(ch, m * NE + e);
+                    for (int m = 0; m < NCH; ++m) mub[m] += we * ldk(ch, m * NE + e);
+                }
+            } else {  // rays that charge nothing: every exponential is 1
+#pragma unroll 4
+                for (int e = 0; e < NE; ++e) {
+                    const double pe = ldk(pdf, e);
+                    sw += pe;
+#pragma unroll
+                    for (int m = 0; m < NCH; ++m) mub[m] += pe * ldk(ch, m * NE + e);
+                }
+                se = sw;
             }
             double p;
             if (se < 1e-30 * sw) {  // opaque ray: FP64 terms relative to the smallest exponent
-                p = mubar_opaque(acc.L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, NCH);
+                p = mubar_opaque(L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, NCH);
             } else {
                 p = -log(se / sw);
 #pragma unroll
@@ -955,18 +1165,31 @@ __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const fl
         for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = m < nl ? ldg(Ls, (size_t)m * nrays + o) : 0.0f;
         double sw = 0.0, se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
         const float k2 = (float)(-inv_xf * 1.4426950408889634);
-        for (int e = 0; e < NE; ++e) {
-            float tr = 0.0f;
+        if (__any(!all_zero(L))) {
+#pragma unroll 4
+            for (int e = 0; e < NE; ++e) {
+                float tr = 0.0f;
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                if (m < nl) tr = fmaf(ldg(muf, m * NE + e), L[m], tr);
-            const double pe = ldg(pdf, e);
-            const double we = pe * (double)exp2f(tr * k2);
-            sw += pe;
-            se += we;
+                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
+                const double pe = ldk(pdf, e);
+                const double we = pe * (double)exp2f(tr * k2);
+                sw += pe;
+                se += we;
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                if (m < nch) mub[m] += we * ldg(ch, m * NE + e);
+                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    if (m < nch) mub[m] += we * ldk(ch, m * NE + e);
+            }
+        } else {  // rays that charge nothing: every exponential is 1
+#pragma unroll 4
+            for (int e = 0; e < NE; ++e) {
+                const double pe = ldk(pdf, e);
+                sw += pe;
+#pragma unroll
+                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    if (m < nch) mub[m] += pe * ldk(ch, m * NE + e);
+            }
+            se = sw;
         }
         if (se < 1e-30 * sw) {  // opaque ray: FP64 terms relative to the smallest exponent
             (void)mubar_opaque(L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, nch);
@@ -1006,8 +1229,8 @@ __global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_scatter(ProjGeom g
         any = any || sc.c[m] != 0.f;
     }
     if (!__any(any)) return;  // nothing to scatter for this wave (e.g. zero upstream gradient)
-    const double c = ldg(tab, a), sn = ldg(tab, g.nAng + a), xc = ldg(tab, 2 * g.nAng + a),
-                 yc = ldg(tab, 3 * g.nAng + a);
+    const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
+                 yc = ldk(tab, 3 * g.nAng + a);
     traverse_wave(g, c, sn, xc, yc, j, jj, active, sc, steps);
 }
 

@@ -67,6 +67,15 @@ __device__ __forceinline__ T ldg(const T* p, size_t i) {
     __builtin_memcpy(&r, (GT*)p + i, sizeof(T));  // (HIP vector types have no copy from a qualified object)
     return r;
 }
+// A table that no kernel writes while it is read (spectra, angles), at a wave-uniform index: a scalar load.  (Through a
+// global pointer the compiler falls back to vector loads once a kernel's stores are too many for its alias search: the
+// spectral sums then waited for five vector loads per energy bin, 25 ms instead of 18 on the dual-energy
+// coefficients of a 512x512x64 / 360-angle problem.)
+template <class T>
+__device__ __forceinline__ T ldk(const T* p, size_t i) {
+    typedef __attribute__((address_space(4))) const T KT;
+    return ((KT*)p)[i];
+}
 template <class T>
 __device__ __forceinline__ void stg(T* p, size_t i, T v) {
     typedef __attribute__((address_space(1))) T GT;
