@@ -612,8 +612,7 @@ static int run_adjoint(vcbct_projector* p, const float* tg, float* dev_grad, dou
     const size_t nv = vox_count(p->g);
     if (!p->d_grad_vox && dev_malloc((void**)&p->d_grad_vox, nv * 32) != hipSuccess)
         return fail(VCBCT_ENOMEM, "device allocation of the gradient volume failed");
-    const size_t nrays = (size_t)p->g.nAng * p->g.H * p->g.W;
-    if (!p->d_coef && dev_malloc((void**)&p->d_coef, nrays * p->g.nmat * sizeof(float)) != hipSuccess)
+    if (!p->d_coef && dev_malloc((void**)&p->d_coef, adjoint_coef_bytes(p->g)) != hipSuccess)
         return fail(VCBCT_ENOMEM, "device allocation of the adjoint coefficients failed");
     // scatter target [mat][y][x][z] (FP32 planes); zero with a fill kernel, not hipMemsetAsync, so the call
     // stays safe under stream capture
@@ -659,8 +658,7 @@ extern "C" int vcbct_projector_multi_loss_grad(vcbct_projector* p, const float* 
     const size_t nv = vox_count(p->g);
     if (!p->d_grad_vox && dev_malloc((void**)&p->d_grad_vox, nv * 32) != hipSuccess)
         return fail(VCBCT_ENOMEM, "device allocation of the gradient volume failed");
-    const size_t nrays = (size_t)p->g.nAng * p->g.H * p->g.W;
-    if (!p->d_coef && dev_malloc((void**)&p->d_coef, nrays * p->g.nmat * sizeof(float)) != hipSuccess)
+    if (!p->d_coef && dev_malloc((void**)&p->d_coef, adjoint_coef_bytes(p->g)) != hipSuccess)
         return fail(VCBCT_ENOMEM, "device allocation of the adjoint coefficients failed");
     SpecSet ss{};
     for (int s = 0; s < p->nspec_multi; ++s) {
@@ -752,8 +750,7 @@ extern "C" int vcbct_projector_logproj_backward_saved(vcbct_projector* p, const 
     const size_t nv = vox_count(p->g);
     if (!p->d_grad_vox && dev_malloc((void**)&p->d_grad_vox, nv * 32) != hipSuccess)
         return fail(VCBCT_ENOMEM, "device allocation of the gradient volume failed");
-    const size_t nrays = (size_t)p->g.nAng * p->g.H * p->g.W;
-    if (!p->d_coef && dev_malloc((void**)&p->d_coef, nrays * p->g.nmat * sizeof(float)) != hipSuccess)
+    if (!p->d_coef && dev_malloc((void**)&p->d_coef, adjoint_coef_bytes(p->g)) != hipSuccess)
         return fail(VCBCT_ENOMEM, "device allocation of the adjoint coefficients failed");
     rc = launch_zero(p->d_grad_vox, nv * 4 * p->mix.nch, st);
     if (rc) return rc;

@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
         }
 #pragma unroll
         for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-            if (m < nch) stg(coef, (size_t)m * nrays + o, (float)(w * mub[m] * inv_xf));
+            if (m < nch) stg(coef, (size_t)m * nrays + ((size_t)a * g.W + jj) * g.H + j, (float)(w * mub[m] * inv_xf));
     }
     if (MODE == VCBCT_ADJ_LOSS && loss) {
         // wave reduction of the loss, one atomic per wave
@@ -1139,7 +1139,8 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(
             for (int m = 0; m < NCH; ++m) cacc[m] += 2.0 * res * mub[m];
         }
 #pragma unroll
-        for (int m = 0; m < NCH; ++m) stg(coef, (size_t)m * nrays + o, (float)(cacc[m] * inv_xf));
+        for (int m = 0; m < NCH; ++m)
+            stg(coef, (size_t)m * nrays + ((size_t)a * g.W + jj) * g.H + j, (float)(cacc[m] * inv_xf));
     }
     if (loss) {
         double v = lossc;
@@ -1150,7 +1151,9 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(
 }
 
 // The coefficients of the upstream-gradient mode from line integrals saved by the forward log projection
-// (the same traversal, so the same FP32 sums): one thread per ray, the epilogue of k_adjoint_coef.
+// (the same traversal, so the same FP32 sums): one thread per ray, the epilogue of k_adjoint_coef.  A block takes 16 x 16
+// rays of an angle, so that the reads (along the detector row) and the writes (along the column) both keep to
+// 64-byte runs.
 __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const float* __restrict__ Ls,
                                                             const double* __restrict__ mu,
                                                             const double* __restrict__ pdf,
@@ -1159,7 +1162,13 @@ __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const fl
                                                             double inv_xf, int nl, const float* __restrict__ gp,
                                                             float* __restrict__ coef) {
     const size_t nrays = (size_t)g.nAng * g.H * g.W;
-    for (size_t o = (size_t)blockIdx.x * 256 + threadIdx.x; o < nrays; o += (size_t)gridDim.x * 256) {
+    const int ncb = (g.W + 15) / 16, nrb = (g.H + 15) / 16;
+    for (size_t b = blockIdx.x; b < (size_t)g.nAng * ncb * nrb; b += gridDim.x) {
+        const int a = (int)(b / ((size_t)ncb * nrb)), rc = (int)(b % ((size_t)ncb * nrb));
+        const int jj = rc % ncb * 16 + (threadIdx.x & 15), row = rc / ncb * 16 + (threadIdx.x >> 4);
+        if (jj >= g.W || row >= g.H) continue;
+        const size_t o = ((size_t)a * g.H + row) * g.W + jj;
+        const size_t oc = ((size_t)a * g.W + jj) * g.H + (g.H - 1 - row);
         float L[VCBCT_MAX_MAT];
 #pragma unroll
         for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = m < nl ? ldg(Ls, (size_t)m * nrays + o) : 0.0f;
@@ -1200,29 +1209,24 @@ __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const fl
         const double w = (double)ldg(gp, o);
 #pragma unroll
         for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-            if (m < nch) stg(coef, (size_t)m * nrays + o, (float)(w * mub[m] * inv_xf));
+            if (m < nch) stg(coef, (size_t)m * nrays + oc, (float)(w * mub[m] * inv_xf));
     }
 }
 
+// One wave of the ray-ordered scatter: 64 detector rows [64 rg, 64 rg + 64) of column jj at angle a.
 template <int NCH>
-__global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_scatter(ProjGeom g, const double* __restrict__ tab,
-                                                                     TileMap tm, const float* __restrict__ coef,
-                                                                     float* __restrict__ gvox) {
-    __shared__ WaveLds step_tabs[4];
-    WaveLds* steps = &step_tabs[threadIdx.x >> 6];
-    const Tile t = tile_map(tm, g.nAng);
+__device__ __forceinline__ void scatter_wave(const ProjGeom& g, const double* __restrict__ tab, int a, int rg, int jj,
+                                             const float* __restrict__ coef, float* __restrict__ gvox,
+                                             WaveLds* steps) {
     const int lane = threadIdx.x & 63;
-    const int j = t.rg * 64 + lane;
-    const int jj = t.col;
-    const int a = t.a;
-    if (jj >= g.W || a >= g.nAng || t.rg * 64 >= g.H) return;  // wave out of range: uniform exit
+    const int j = rg * 64 + lane;
     const bool active = j < g.H;
     ScatterG<NCH> sc;  // the scattered channels: the maps, or their spectral basis
     sc.gvox = gvox;
     sc.plane = (size_t)g.N * g.N * g.Nz;
     bool any = false;
     const size_t nrays = (size_t)g.nAng * g.H * g.W;
-    const size_t o = (size_t)a * g.H * g.W + (size_t)(g.H - 1 - (active ? j : 0)) * g.W + jj;
+    const size_t o = ((size_t)a * g.W + jj) * g.H + (active ? j : 0);
 #pragma unroll
     for (int m = 0; m < NCH; ++m) {
         sc.c[m] = active ? ldg(coef, (size_t)m * nrays + o) : 0.f;
@@ -1232,6 +1236,32 @@ __global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_scatter(ProjGeom g
     const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
                  yc = ldk(tab, 3 * g.nAng + a);
     traverse_wave(g, c, sn, xc, yc, j, jj, active, sc, steps);
+}
+
+template <int NCH>
+__global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_scatter(ProjGeom g, const double* __restrict__ tab,
+                                                                     TileMap tm, const float* __restrict__ coef,
+                                                                     float* __restrict__ gvox) {
+    __shared__ WaveLds step_tabs[4];
+    const Tile t = tile_map(tm, g.nAng);
+    if (t.col >= g.W || t.a >= g.nAng || t.rg * 64 >= g.H) return;  // wave out of range: uniform exit
+    scatter_wave<NCH>(g, tab, t.a, t.rg, t.col, coef, gvox, &step_tabs[threadIdx.x >> 6]);
+}
+
+// The ray-ordered scatter of the columns that the tile form leaves over: listed[0] of them, from listed[4] on.
+template <int NCH>
+__global__ __launch_bounds__(256) VCBCT_WAVES8 void k_adjoint_scatter_listed(ProjGeom g,
+                                                                            const double* __restrict__ tab,
+                                                                            const int* __restrict__ listed,
+                                                                            const float* __restrict__ coef,
+                                                                            float* __restrict__ gvox) {
+    __shared__ WaveLds step_tabs[4];
+    const int wave = threadIdx.x >> 6, nrg = (g.H + 63) / 64;
+    const int n = __builtin_amdgcn_readfirstlane(listed[0]);
+    for (long i = (long)blockIdx.x * 4 + wave; i < (long)n * nrg; i += (long)gridDim.x * 4) {
+        const int e = __builtin_amdgcn_readfirstlane(listed[4 + i / nrg]);
+        scatter_wave<NCH>(g, tab, e / g.W, (int)(i % nrg), e % g.W, coef, gvox, &step_tabs[wave]);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1587,6 +1617,24 @@ static int launch_scatter(const ProjGeom& g, const double* tables, const float* 
     return 0;
 }
 
+static int launch_scatter_listed(const ProjGeom& g, const double* tables, const int* listed, const float* coef,
+                                 int nch, float* grad_vox, hipStream_t st) {
+#define VCBCT_LAUNCH_LISTED(C)                                                                                  \
+    hipLaunchKernelGGL(k_adjoint_scatter_listed<C>, dim3(512), dim3(256), 0, st, g, tables, listed, coef, grad_vox)
+    switch (nch) {
+        case 1: VCBCT_LAUNCH_LISTED(1); break;
+        case 2: VCBCT_LAUNCH_LISTED(2); break;
+        case 3: VCBCT_LAUNCH_LISTED(3); break;
+        case 4: VCBCT_LAUNCH_LISTED(4); break;
+        case 5: VCBCT_LAUNCH_LISTED(5); break;
+        case 6: VCBCT_LAUNCH_LISTED(6); break;
+        default: return fail(VCBCT_EINVAL, "adjoint: %d channels", nch);
+    }
+#undef VCBCT_LAUNCH_LISTED
+    VCBCT_HIP(hipGetLastError());
+    return 0;
+}
+
 // The shape of an adjoint kernel: the caller's (forced.rgb > 0, 4 waves), else the tuned one for `key`, tuned
 // now with `launch` if there is none.
 template <class F>
@@ -1617,13 +1665,34 @@ static int scatter_shape(const ProjGeom& g, const double* tables, const float* c
     return launch_zero(grad_vox, (size_t)nch * g.N * g.N * g.Nz * sizeof(float), st);
 }
 
+size_t adjoint_coef_bytes(const ProjGeom& g) {
+    return align16((size_t)g.nAng * g.H * g.W * g.nmat * sizeof(float)) + (scatter_by_tiles(g) ? scatter_work_bytes(g) : 0);
+}
+
+// The gradient's channel planes from the coefficients: by voxel tiles (scatter.hip) and the columns that form leaves
+// over, or ray by ray where the caller fixed that form's shape or the geometry is outside the tile form's range.
+static int run_scatter(const ProjGeom& g, const double* tables, float* coef, int nch, float* grad_vox, hipStream_t st,
+                       const TileShape& forced) {
+    if (forced.rgb > 0 || !scatter_by_tiles(g)) {
+        TileShape s;
+        int rc = scatter_shape(g, tables, coef, nch, grad_vox, st, forced, s);
+        return rc ? rc : launch_scatter(g, tables, coef, nch, grad_vox, st, s);
+    }
+    void* work = (char*)coef + align16((size_t)g.nAng * g.H * g.W * g.nmat * sizeof(float));
+    const int* listed = nullptr;
+    int rc = launch_scatter_rays(g, tables, work, st, &listed);
+    if (!rc) rc = launch_scatter_tiles(g, tables, work, coef, nch, grad_vox, st);
+    if (!rc) rc = launch_scatter_listed(g, tables, listed, coef, nch, grad_vox, st);
+    return rc;
+}
+
 int launch_adjoint(const ProjGeom& g, const double* tables, const void* vox, int vox_kind, const Spectrum& sp,
                    double xfactor, const float* target_or_gp, int mode, float* coef, float* grad_vox, double* loss,
                    hipStream_t st, const TileShape& forced) {
     const double inv_xf = 1.0 / xfactor;
     char extra[64];
     snprintf(extra, sizeof extra, "mode%d nch%d NE%d %s", mode, sp.nch, sp.NE, vox_name(vox_kind));
-    TileShape sc, ss;
+    TileShape sc;
     bool tuned_now = false;
     // tuning launches pass no loss accumulator
     auto launch = [&](const TileShape& t) {
@@ -1631,9 +1700,7 @@ int launch_adjoint(const ProjGeom& g, const double* tables, const void* vox, int
     };
     int rc = adjoint_shape(forced, tune_key("adj-coef", g, g.nAng, extra), st, launch, sc, tuned_now);
     if (!rc) rc = launch_coef(g, tables, vox, vox_kind, sp, inv_xf, target_or_gp, mode, coef, loss, st, sc);
-    if (!rc) rc = scatter_shape(g, tables, coef, sp.nch, grad_vox, st, forced, ss);
-    if (!rc) rc = launch_scatter(g, tables, coef, sp.nch, grad_vox, st, ss);
-    return rc;
+    return rc ? rc : run_scatter(g, tables, coef, sp.nch, grad_vox, st, forced);
 }
 
 int launch_adjoint_multi(const ProjGeom& g, const double* tables, const void* vox, int vox_kind, const SpecSet& ss,
@@ -1644,30 +1711,25 @@ int launch_adjoint_multi(const ProjGeom& g, const double* tables, const void* vo
     int ne = 0;
     for (int s = 0; s < ss.nspec; ++s) ne += ss.NE[s];
     snprintf(extra, sizeof extra, "nspec%d nch%d NE%d %s", ss.nspec, ss.nch, ne, vox_name(vox_kind));
-    TileShape sc, sg;
+    TileShape sc;
     bool tuned_now = false;
     auto launch = [&](const TileShape& t) {
         return launch_coef_multi(g, tables, vox, vox_kind, ss, inv_xf, targets, coef, nullptr, st, t);
     };
     int rc = adjoint_shape(forced, tune_key("adj-multi", g, g.nAng, extra), st, launch, sc, tuned_now);
     if (!rc) rc = launch_coef_multi(g, tables, vox, vox_kind, ss, inv_xf, targets, coef, loss, st, sc);
-    if (!rc) rc = scatter_shape(g, tables, coef, ss.nch, grad_vox, st, forced, sg);
-    if (!rc) rc = launch_scatter(g, tables, coef, ss.nch, grad_vox, st, sg);
-    return rc;
+    return rc ? rc : run_scatter(g, tables, coef, ss.nch, grad_vox, st, forced);
 }
 
 int launch_adjoint_saved(const ProjGeom& g, const double* tables, const float* Ls, const Spectrum& sp,
                          double xfactor, const float* gp, float* coef, float* grad_vox, hipStream_t st,
                          const TileShape& forced) {
-    const size_t nrays = (size_t)g.nAng * g.H * g.W;
-    const unsigned nbc = (unsigned)std::min<size_t>((nrays + 255) / 256, 65536);
+    const unsigned nbc =
+        (unsigned)std::min<size_t>((size_t)g.nAng * ((g.H + 15) / 16) * ((g.W + 15) / 16), 65536);
     hipLaunchKernelGGL(k_adjoint_coef_saved, dim3(nbc), dim3(256), 0, st, g, Ls, sp.mu, sp.pdf, sp.muf, sp.ch, sp.nch,
                        sp.NE, 1.0 / xfactor, sp.nl, gp, coef);
     VCBCT_HIP(hipGetLastError());
-    TileShape sg;
-    int rc = scatter_shape(g, tables, coef, sp.nch, grad_vox, st, forced, sg);
-    if (!rc) rc = launch_scatter(g, tables, coef, sp.nch, grad_vox, st, sg);
-    return rc;
+    return run_scatter(g, tables, coef, sp.nch, grad_vox, st, forced);
 }
 
 }  // namespace vcbct

@@ -218,6 +218,18 @@ int launch_adjoint_multi(const ProjGeom& g, const double* tables, const void* vo
                          double xfactor, const float* targets, float* coef, float* grad_vox, double* loss,
                          hipStream_t st, const TileShape& forced);
 
+// Size of the adjoint's coefficient buffer: a coefficient per ray and map ([channel][angle][column][row], rows in the
+// kernels' order, so that the rows of a wave are contiguous), and the tile scatter's workspace behind them.
+inline size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
+size_t adjoint_coef_bytes(const ProjGeom& g);
+// The scatter by voxel tiles (scatter.hip): whether it serves the geometry, its workspace, the rays' paths (with the
+// list of columns left to the ray-ordered scatter: listed[0] of them, from listed[4] on) and the scatter itself.
+bool scatter_by_tiles(const ProjGeom& g);
+size_t scatter_work_bytes(const ProjGeom& g);
+int launch_scatter_rays(const ProjGeom& g, const double* tables, void* work, hipStream_t st, const int** listed);
+int launch_scatter_tiles(const ProjGeom& g, const double* tables, const void* work, const float* coef, int nch,
+                         float* gvox, hipStream_t st);
+
 // a / b for a divisor b known in advance, with rb = 1 / b correctly rounded: the product a * rb is within an
 // ulp of a / b, and one correction with the exact remainder a - q b (an FMA) rounds it correctly (Markstein's
 // theorem, round-to-nearest, no overflow or underflow), so the result equals the IEEE quotient bit for bit in
@@ -286,7 +298,7 @@ struct vcbct_projector {
     uint16_t* d_vox_u16;   // [N][N][Nz][8] (y, x, z, mat)
     float* d_vox_f32;      // [N][N][Nz][8]
     float* d_grad_vox;     // adjoint scatter target, planar [mat][y][x][z]
-    float* d_coef;         // adjoint per-ray coefficients [mat][angle][row][col]
+    float* d_coef;         // adjoint per-ray coefficients [mat][angle][col][row], then the tile scatter's workspace
     void* d_lp_tab;        // lengthproj per-angle constants (two forms, see iterative.hip)
     double* d_mu;          // [nmat][NE]
     double* d_pdf;         // [NE]
