@@ -504,37 +504,40 @@ __global__ __launch_bounds__(256) void k_backproject(float* __restrict__ recon, 
 }
 
 
-// The same backprojection with the projection data staged in LDS.  Per angle, the rows and columns that the
-// block's 16 x 16 columns and ZB slices can sample (its footprint on the panel) are loaded into an LDS tile by
-// the whole block, coalesced along the rows, and the taps are read from the tile.  The footprint's columns
-// come from a per-(block, angle) table built with the plan: U is a linear-fractional function of (x, y), so
-// over the block's square its extremes lie at the four corner voxels; the base column floor(W/2 + U + xs -
-// 0.5) is taken there in the same FP64 expression, widened by one column before and two after.  Its rows
-// come from the extremes of 1 / (L2 pitch) at the corners (also in the table) and the block's slice range,
-// widened likewise.  A tap outside the tile (a footprint larger than the tile, or a rounding beyond the
-// margins) is read from global memory at the address the unstaged kernel reads, so the result is identical
-// to k_backproject's bit for bit.  Two tiles alternate, so one barrier per angle suffices: a tile is
-// rewritten two angles after it was read, and every thread has passed the barrier in between.
-struct BpFoot {
-    int u0, u1;      // columns [u0, u1] of the footprint (clamped to the panel; u0 > u1: none)
-    float ilo, ihi;  // extremes of (1 / L2) / pitch over the block's corner voxels
-};
-constexpr int BP_TILE = 2048;  // floats per staged tile (8 KB; two per block)
+// The same backprojection with the projections staged in LDS.  A block is 8 x 8 voxel columns by 4 ZB slices; its four
+// waves take the same columns and ZB slices each, and go through the angles four at a time.  Each wave prepares one of
+// the next four while it backprojects the current ones:
+//  - the columns' geometry (weights and base column in the same FP64 expressions as above), handed to all four waves
+//    through LDS, which leaves those ~50 instructions per angle to 4 ZB slices instead of ZB;
+//  - the part of the projection that the block samples (BP_TC columns by TR rows at most), loaded along the rows into
+//    registers and written to LDS after the current angles.
+// U and 1 / L2 are linear-fractional in (x, y), so their extremes over the block are at its four corner columns, and the
+// footprint is theirs, widened by more than a rounding.  An angle whose footprint leaves the panel, or the tile, goes
+// through the loads, clamps and selects of k_backproject.  Two sets of buffers alternate: one barrier per four angles.
+// k_backproject is bound by its taps in the vector L1 (~20 cycles per two-word load of a wave: 2.7 ms on 270x270x128 / 360
+// angles of 400x400); from LDS they are two paired reads, and the kernel is bound by vector issue (~17 instructions an
+// update, 11 of them the interpolation): 1.68 ms with 8 slices a thread, 1.77 with 4.
+// Eight slices a thread span up to 58 rows there, four 30.  The taller tile has one buffer (and a second barrier), so
+// that four blocks fit a CU's 160 KB either way.
+constexpr int BP_TC = 32;
 
 template <int ZB>
 __global__ __launch_bounds__(256) void k_backproject_lds(float* __restrict__ recon, const float* __restrict__ sino,
                                                          int R, int Z, double zstart, double step, double scale,
                                                          int H, int W, int n, const double* __restrict__ atab,
-                                                         double xfactor, double pitchW,
-                                                         const BpFoot* __restrict__ foot) {
-    __shared__ float tiles[2][BP_TILE];
-    const int x = blockIdx.x * 16 + (threadIdx.x & 15);
-    const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
-    const int z0 = blockIdx.z * ZB;
+                                                         double xfactor, double pitchW) {
+    __shared__ float4 geom[2][4][64];  // wf, iL, wgt, byte offset of the base column (in the tile, or the panel; < 0: none)
+    constexpr int TR = ZB == 8 ? 58 : 30, NT = ZB == 8 ? 1 : 2;
+    __shared__ float tile[NT][4][TR * BP_TC];
+    __shared__ int staged[2][4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = blockIdx.x * 8 + (lane & 7);
+    const int y = blockIdx.y * 8 + (lane >> 3);
+    const int zb0 = blockIdx.z * (4 * ZB), z0 = zb0 + wave * ZB;
     const double rad = (double)(R - 1) / 2.0;
-    // every thread stages and meets the barriers; only the voxels inside the mask accumulate
     const bool active = x < R && y < R &&
                         ((double)y - rad) * ((double)y - rad) + ((double)x - rad) * ((double)x - rad) <= rad * rad;
+    if (!__any(active)) return;  // (the same columns, so the same answer, in all four waves)
     const double centerPos = (double)R / 2.0 - 0.5;
     const double xx = (x - centerPos) * scale;
     const double yy = -(y - centerPos) * scale;
@@ -545,30 +548,22 @@ __global__ __launch_bounds__(256) void k_backproject_lds(float* __restrict__ rec
         zz[i] = (float)(zstart + (double)(z0 + i) * step);
         acc[i] = 0.f;
     }
+    const float zlo = (float)(zstart + (double)zb0 * step), zhi = (float)(zstart + (double)(zb0 + 4 * ZB - 1) * step);
     const double hW = (double)(W / 2);
     const float hH = (float)(H / 2);
     const float ipW = (float)(1.0 / pitchW);
     const double rpW = 1.0 / pitchW;  // correctly rounded: the divisions by pitchW below are exact products
-    const BpFoot* fb = foot + (size_t)(blockIdx.y * gridDim.x + blockIdx.x) * n;
-    const float zlo = zz[0], zhi = zz[ZB - 1];
-    for (int th = 0; th < n; ++th) {
-        const BpFoot f = fb[th];
-        const float e0 = zlo * f.ilo, e1 = zlo * f.ihi, e2 = zhi * f.ilo, e3 = zhi * f.ihi;
-        const int r0 = max(0, (int)floorf(hH + fminf(fminf(e0, e1), fminf(e2, e3))) - 1);
-        const int r1 = min(H - 1, (int)floorf(hH + fmaxf(fmaxf(e0, e1), fmaxf(e2, e3))) + 2);
-        const int tw = f.u1 - f.u0 + 1, tr = r1 - r0 + 1;
-        const bool use_tile = tw > 0 && tr > 0 && tw * tr <= BP_TILE;  // uniform over the block
-        float* tile = tiles[th & 1];
-        const float* P = sino + (size_t)th * H * W;
-        if (use_tile) {
-            for (int i = threadIdx.x; i < tw * tr; i += 256) {
-                const int rr = i / tw, cc = i - rr * tw;
-                tile[i] = P[(size_t)(r0 + rr) * W + f.u0 + cc];
-            }
-        }
-        __syncthreads();
-        if (!active) continue;
-        const double c = atab[th], s = atab[n + th], dbeta = atab[2 * n + th], xs = atab[3 * n + th];
+    const int rowb = W * 4;
+    const float hm1 = (float)(H - 1);
+    float px[TR / 2];  // the next tile's pixels: row 2 i + lane / 32, column lane % 32
+    bool fits = false;
+
+    // prepares the wave's angle of the four from th0 on: geometry to LDS, pixels on their way to px
+    auto form = [&](int th0, int buf) {
+        const int th = th0 + wave;
+        if (th >= n) return;
+        const double c = ldk(atab, th), s = ldk(atab, n + th), dbeta = ldk(atab, 2 * n + th),
+                     xs = ldk(atab, 3 * n + th);
         double X = xx * c + yy * s;
         double Y = -xx * s + yy * c;
         double L2 = 1.0 - div_known(Y, 100.0, 0.01);  // = 1.0 - Y / 100.0 bit for bit
@@ -578,82 +573,89 @@ __global__ __launch_bounds__(256) void k_backproject_lds(float* __restrict__ rec
         double w = U - fU;
         int UU = (int)floor(hW + U + xs - 0.5);
         const bool ucol = (UU >= 0 && UU < W - 1), uedge = (UU == W - 1);
-        if (!ucol && !uedge) continue;
         const float rL2 = __builtin_amdgcn_rcpf((float)L2);
         const float iL = rL2 * ipW;
         const float wgt = rL2 * rL2 * (float)(dbeta * xfactor);
-        const float wf = (float)w;
-        auto tap = [&](int r, int col) -> float {
-            const int a = r - r0, b = col - f.u0;
-            return (use_tile && (unsigned)a < (unsigned)tr && (unsigned)b < (unsigned)tw) ? tile[a * tw + b]
-                                                                                      : P[(size_t)r * W + col];
-        };
+        const float wf = ucol ? (float)w : 0.f;  // (the last column: weight 0, as in k_backproject)
+        // the footprint, from the corner columns (iL > 0, so its bits order as integers)
+        const int li = __builtin_bit_cast(int, iL);
+        const int ua = __builtin_amdgcn_readlane(UU, 0), ub = __builtin_amdgcn_readlane(UU, 7);
+        const int uc = __builtin_amdgcn_readlane(UU, 56), ud = __builtin_amdgcn_readlane(UU, 63);
+        const int la = __builtin_amdgcn_readlane(li, 0), lb = __builtin_amdgcn_readlane(li, 7);
+        const int lc = __builtin_amdgcn_readlane(li, 56), ld = __builtin_amdgcn_readlane(li, 63);
+        const int u0 = min(min(ua, ub), min(uc, ud)) - 1, u1 = max(max(ua, ub), max(uc, ud)) + 2;
+        const float ilo = __builtin_bit_cast(float, min(min(la, lb), min(lc, ld)));
+        const float ihi = __builtin_bit_cast(float, max(max(la, lb), max(lc, ld)));
+        const float elo = hH + fminf(zlo, zhi) * (fminf(zlo, zhi) < 0.f ? ihi : ilo);
+        const float ehi = hH + fmaxf(zlo, zhi) * (fmaxf(zlo, zhi) < 0.f ? ilo : ihi);
+        const int r0 = __builtin_amdgcn_readfirstlane((int)floorf(fmaxf(elo - 0.01f, -2.f)));
+        const int r1 = __builtin_amdgcn_readfirstlane((int)floorf(fminf(ehi + 0.01f, hm1 + 1.f)) + 1);
+        // (a volume that reaches the source's distance, where 1 / L2 has no bounds, is not staged)
+        fits = min(min(la, lb), min(lc, ld)) > 0 && ihi < 1.0e4f && r0 >= 0 && r1 <= H - 1 && r1 - r0 < TR && u1 - u0 < BP_TC && __all(!active || ucol || uedge);
+        const int off = fits ? (UU - u0) * 4 - r0 * (BP_TC * 4) : ucol || uedge ? UU * 4 : INT_MIN;
+        geom[buf][wave][lane] = make_float4(wf, iL, wgt, __builtin_bit_cast(float, off));
+        if (lane == 0) staged[buf][wave] = fits;
+        if (fits) {
+            const __amdgpu_buffer_rsrc_t P = bp_rsrc(sino + (size_t)th * H * W, H * W * 4);
+            const int vo = ((r0 + (lane >> 5)) * W + u0 + (lane & 31)) * 4;  // (columns off the panel: never sampled)
 #pragma unroll
-        for (int i = 0; i < ZB; ++i) {
-            const float ZETA = fmaf(zz[i], iL, hH);
-            const float fz = floorf(ZETA);
-            const int NZ = (int)fz;
-            const float wz = ZETA - fz;
-            float sum;
-            if (NZ >= 0 && NZ < H - 1) {
-                if (ucol) {
-                    float a0 = tap(NZ, UU), a1 = tap(NZ, UU + 1), b0 = tap(NZ + 1, UU), b1 = tap(NZ + 1, UU + 1);
-                    sum = bp_lerp(bp_lerp(a0, a1, wf), bp_lerp(b0, b1, wf), wz);
-                } else {
-                    sum = bp_lerp(tap(NZ, UU), tap(NZ + 1, UU), wz);
-                }
-            } else if (NZ == H - 1) {
-                sum = ucol ? bp_lerp(tap(NZ, UU), tap(NZ, UU + 1), wf) : tap(NZ, UU);
-            } else {
-                continue;
-            }
-            acc[i] = fmaf(sum, wgt, acc[i]);
+            for (int i = 0; i < TR / 2; ++i)
+                if (r0 + 2 * i <= r1) px[i] = bp_ld(P, vo, 2 * i * rowb);
         }
+    };
+    auto put = [&](int buf) {
+        if (NT == 1) __syncthreads();
+        if (!fits) return;
+#pragma unroll
+        for (int i = 0; i < TR / 2; ++i) tile[buf % NT][wave][i * 64 + lane] = px[i];
+    };
+    form(0, 0);
+    put(0);
+    int buf = 0;
+    for (int th0 = 0; th0 < n; th0 += 4, buf ^= 1) {
+        __syncthreads();
+        fits = false;
+        form(th0 + 4, buf ^ 1);  // (those buffers' last readers passed the barrier above)
+        const int nk = min(4, n - th0);
+        for (int k = 0; k < nk; ++k) {
+            const float4 q = geom[buf][k][lane];
+            const float wf = q.x, iL = q.y, wgt = q.z;
+            const int off = __builtin_bit_cast(int, q.w);
+            if (__builtin_amdgcn_readfirstlane(staged[buf][k])) {
+                const char* T = (const char*)tile[buf % NT][k] + off;
+#pragma unroll
+                for (int i = 0; i < ZB; ++i) {
+                    const float ZETA = fmaf(zz[i], iL, hH);
+                    const float wz = __builtin_amdgcn_fractf(ZETA);  // (ZETA >= 0: = ZETA - floor(ZETA))
+                    const float* t = (const float*)(T + ((int)ZETA << 7));
+                    const float h0 = bp_lerp(t[0], t[1], wf), h1 = bp_lerp(t[BP_TC], t[BP_TC + 1], wf);
+                    acc[i] = fmaf(bp_lerp(h0, h1, wz), wgt, acc[i]);
+                }
+            } else {
+                const bool inpanel = off >= 0;
+                const unsigned UU4 = inpanel ? (unsigned)off : 0u;
+                const __amdgpu_buffer_rsrc_t P = bp_rsrc(sino + (size_t)(th0 + k) * H * W, H * W * 4);
+#pragma unroll
+                for (int i = 0; i < ZB; ++i) {
+                    const float ZETA = fmaf(zz[i], iL, hH);
+                    const float fz = floorf(ZETA);
+                    const float wz = ZETA - fz;
+                    const float fzc = __builtin_amdgcn_fmed3f(fz, 0.f, hm1);
+                    const int vo = (int)(__umul24((unsigned)(int)fzc, (unsigned)rowb) + UU4);
+                    const float a0 = bp_ld(P, vo, 0), a1 = bp_ld(P, vo + 4, 0);
+                    const float b0 = bp_ld(P, vo, rowb), b1 = bp_ld(P, vo + 4, rowb);
+                    const float h0 = bp_lerp(a0, a1, wf), h1 = bp_lerp(b0, b1, wf);
+                    const float sum = fz < hm1 ? bp_lerp(h0, h1, wz) : h0;
+                    acc[i] = fmaf((inpanel && fzc == fz) ? sum : 0.f, wgt, acc[i]);
+                }
+            }
+        }
+        put(buf ^ 1);
     }
     if (!active) return;
 #pragma unroll
     for (int i = 0; i < ZB; ++i)
         if (z0 + i < Z) recon[((size_t)(z0 + i) * R + y) * R + x] += acc[i];
-}
-
-// Footprint table of the staged backprojector: per (16 x 16 column block, angle), in block-row order.
-static std::vector<BpFoot> bp_foot_table(int R, int W, int n, double scale, double pitch_iso, const double* tab) {
-    const int nb = (R + 15) / 16;
-    const double pitchW = pitch_iso * 800 / W;
-    const double hW = (double)(W / 2);
-    const float ipW = (float)(1.0 / pitchW);
-    const double centerPos = (double)R / 2.0 - 0.5;
-    std::vector<BpFoot> f((size_t)nb * nb * n);
-    for (int by = 0; by < nb; ++by)
-        for (int bx = 0; bx < nb; ++bx)
-            for (int th = 0; th < n; ++th) {
-                const double c = tab[th], s = tab[n + th], xs = tab[3 * n + th];
-                int umin = INT_MAX, umax = INT_MIN;
-                float ilo = 1e30f, ihi = -1e30f;
-                for (int cy = 0; cy < 2; ++cy)
-                    for (int cx = 0; cx < 2; ++cx) {
-                        const int x = cx ? std::min(bx * 16 + 15, R - 1) : bx * 16;
-                        const int y = cy ? std::min(by * 16 + 15, R - 1) : by * 16;
-                        const double xx = (x - centerPos) * scale;
-                        const double yy = -(y - centerPos) * scale;
-                        double X = xx * c + yy * s;
-                        double Y = -xx * s + yy * c;
-                        double L2 = 1.0 - Y / 100.0;
-                        double U = X / L2 / pitchW;
-                        const int UU = (int)floor(hW + U + xs - 0.5);
-                        umin = std::min(umin, UU);
-                        umax = std::max(umax, UU);
-                        const float iL = (1.0f / (float)L2) * ipW;
-                        ilo = std::min(ilo, iL);
-                        ihi = std::max(ihi, iL);
-                    }
-                BpFoot& e = f[((size_t)by * nb + bx) * n + th];
-                e.u0 = std::max(0, umin - 1);
-                e.u1 = std::min(W - 1, umax + 2);
-                e.ilo = ilo;
-                e.ihi = ihi;
-            }
-    return f;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -730,11 +732,12 @@ static int launch_filter(const FilterPlan* P, int H, int W, int n, const float* 
     return 0;
 }
 
-// zb: slices per thread; d_foot non-null: the LDS-staged form with that footprint table.
+// zb: slices per thread; staged: the LDS-staged form.
 static int launch_bp(int zb, int R, int Z, int zstart, double step, double scale, float* drec, int H, int W, int n,
                      const float* ds, const double* d_atab, int xfactor, double pitch_iso, hipStream_t st,
-                     const BpFoot* d_foot = nullptr) {
-    dim3 grid((R + 15) / 16, (R + 15) / 16, (Z + zb - 1) / zb);
+                     bool staged) {
+    const dim3 grid = staged ? dim3((R + 7) / 8, (R + 7) / 8, (Z + 4 * zb - 1) / (4 * zb))
+                             : dim3((R + 15) / 16, (R + 15) / 16, (Z + zb - 1) / zb);
     const double pitchW = pitch_iso * 800 / W;
     // the taps' 24-bit row multiply and 32-bit byte offsets within one projection
     if (H >= (1 << 24) || W >= (1 << 22) || (long long)H * W * 4 >= (1ll << 31))
@@ -744,8 +747,8 @@ static int launch_bp(int zb, int R, int Z, int zstart, double step, double scale
                        d_atab, (double)xfactor, pitchW)
 #define VCBCT_BPL(ZBV)                                                                                                 \
     hipLaunchKernelGGL(k_backproject_lds<ZBV>, grid, dim3(256), 0, st, drec, ds, R, Z, (double)zstart, step, scale, H, \
-                       W, n, d_atab, (double)xfactor, pitchW, d_foot)
-    if (d_foot) {
+                       W, n, d_atab, (double)xfactor, pitchW)
+    if (staged) {
         if (zb == 2) VCBCT_BPL(2);
         else if (zb == 8) VCBCT_BPL(8);
         else VCBCT_BPL(4);
@@ -758,6 +761,15 @@ static int launch_bp(int zb, int R, int Z, int zstart, double step, double scale
 #undef VCBCT_BPL
     VCBCT_HIP(hipGetLastError());
     return 0;
+}
+
+// Whether four slices a thread of the staged form fit their tiles: the rows and columns that a block can sample where the
+// volume comes nearest to the source (1 / L2 largest).  For calls that cannot time the forms; below 16 slices its
+// blocks would be partly empty.  (270x270x64 / 36 angles, one-shot: 222 us staged, 244 plain.)
+static bool bp_staged_fits(int R, int Z, double step, double scale, int W, double pitch_iso) {
+    const double near_l2 = 1.0 - 0.5 * R * scale / 100.0, pix = pitch_iso * 800 / W;
+    return Z >= 16 && near_l2 > 0.1 && 15.0 * step / (near_l2 * pix) + 3.0 <= 30.0 &&
+           7.0 * 1.4143 * scale / (near_l2 * pix) + 5.0 <= BP_TC;
 }
 
 // Autotuner cache: slices per thread of the backprojector, per (R, Z, n, H, W).
@@ -777,9 +789,8 @@ struct vcbct_fdk_plan {
     // it, weighted inside the filter's load with the exponents d_ecol [n][hf_W]
     int hf_W, hf_off;
     float* d_ecol;
-    // backprojector form: LDS-staged (with its footprint table) or not, picked with zb by the autotuner
+    // backprojector form: LDS-staged or not, picked with zb by the autotuner
     int bp_lds;
-    vcbct::BpFoot* d_foot;
 };
 
 namespace vcbct {
@@ -788,8 +799,9 @@ static int tune_bp(vcbct_fdk_plan* p) {
     // VCBCT_BP_LDS=0 / 1 restricts the candidates to the unstaged / LDS-staged form
     const char* lds_env = getenv("VCBCT_BP_LDS");
     const int lds_only = (lds_env && (*lds_env == '0' || *lds_env == '1')) ? *lds_env - '0' : -1;
-    char key[160];
-    snprintf(key, sizeof key, "bp R%d Z%d n%d H%d W%d lds%d", p->R, p->Z, p->n, p->H, p->W, lds_only);
+    char key[224];
+    snprintf(key, sizeof key, "bp R%d Z%d n%d H%d W%d step%.6g scale%.6g pitch%.6g lds%d", p->R, p->Z, p->n, p->H, p->W,
+             p->step, p->scale, p->pitch, lds_only);
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_bp_zb.find(key);
@@ -802,7 +814,7 @@ static int tune_bp(vcbct_fdk_plan* p) {
     const char* off = getenv("VCBCT_NO_AUTOTUNE");
     if (off && *off == '1') {
         p->zb = 4;
-        p->bp_lds = lds_only == 1 ? 1 : 0;
+        p->bp_lds = lds_only >= 0 ? lds_only : bp_staged_fits(p->R, p->Z, p->step, p->scale, p->W, p->pitch);
         return 0;
     }
     float *ds = nullptr, *dr = nullptr;
@@ -821,16 +833,15 @@ static int tune_bp(vcbct_fdk_plan* p) {
     std::string rep = std::string(key) + ":";
     for (int lds = 0; lds < 2; ++lds) {
         if (lds_only >= 0 && lds != lds_only) continue;
-        const BpFoot* foot = lds ? p->d_foot : nullptr;
         for (int zb : {2, 4, 8}) {
             if (rc) break;
             rc = launch_bp(zb, p->R, p->Z, p->zstart, p->step, p->scale, dr, p->H, p->W, p->n, ds, p->d_atab,
-                           p->xfactor, p->pitch, nullptr, foot);  // warm
+                           p->xfactor, p->pitch, nullptr, lds != 0);  // warm
             float ms = 0;
             (void)hipEventRecord(e0, nullptr);
             for (int r = 0; r < 2 && !rc; ++r)
                 rc = launch_bp(zb, p->R, p->Z, p->zstart, p->step, p->scale, dr, p->H, p->W, p->n, ds, p->d_atab,
-                               p->xfactor, p->pitch, nullptr, foot);
+                               p->xfactor, p->pitch, nullptr, lds != 0);
             (void)hipEventRecord(e1, nullptr);
             (void)hipEventSynchronize(e1);
             (void)hipEventElapsedTime(&ms, e0, e1);
@@ -883,18 +894,10 @@ extern "C" int vcbct_fdk_plan_create(vcbct_fdk_plan** out, int H, int W, int n, 
     if (!rc && (hipMemcpy(p->d_ctab, ct.data(), ct.size() * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(p->d_atab, at.data(), at.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess))
         rc = fail(VCBCT_EHIP, "fdk plan upload");
-    if (!rc) {  // footprint table of the LDS-staged backprojector
-        std::vector<BpFoot> ft = bp_foot_table(R, W, n, scale, pitch_iso, at.data());
-        if (dev_malloc((void**)&p->d_foot, ft.size() * sizeof(BpFoot)) != hipSuccess)
-            rc = fail(VCBCT_ENOMEM, "fdk plan footprint table");
-        else if (hipMemcpy(p->d_foot, ft.data(), ft.size() * sizeof(BpFoot), hipMemcpyHostToDevice) != hipSuccess)
-            rc = fail(VCBCT_EHIP, "fdk plan upload");
-    }
     if (!rc) rc = tune_bp(p);
     if (rc) {
         (void)hipFree(p->d_ctab);
         (void)hipFree(p->d_atab);
-        (void)hipFree(p->d_foot);
         free(p);
         return rc;
     }
@@ -953,7 +956,6 @@ extern "C" void vcbct_fdk_plan_destroy(vcbct_fdk_plan* p) {
     if (!p) return;
     (void)hipSetDevice(p->device);
     (void)hipFree(p->d_ecol);
-    (void)hipFree(p->d_foot);
     (void)hipFree(p->d_ctab);
     (void)hipFree(p->d_atab);
     free(p);
@@ -970,7 +972,7 @@ extern "C" int vcbct_fdk_plan_filter(vcbct_fdk_plan* p, const float* dev_proj, f
 extern "C" int vcbct_fdk_plan_backproject(vcbct_fdk_plan* p, const float* dev_filtered, float* dev_recon, void* stream) {
     if (!p || !dev_filtered || !dev_recon) return fail(VCBCT_EINVAL, "fdk_plan_backproject: NULL argument");
     return launch_bp(p->zb, p->R, p->Z, p->zstart, p->step, p->scale, dev_recon, p->H, p->W, p->n, dev_filtered,
-                     p->d_atab, p->xfactor, p->pitch, (hipStream_t)stream, p->bp_lds ? p->d_foot : nullptr);
+                     p->d_atab, p->xfactor, p->pitch, (hipStream_t)stream, p->bp_lds != 0);
 }
 
 extern "C" int vcbct_fdk_plan_bp_staged(const vcbct_fdk_plan* p) { return p ? p->bp_lds : -1; }
@@ -1026,15 +1028,8 @@ extern "C" int vcbct_reconstruct_image(int R, int Z, int zstart, double step, do
     double* d_tab;
     VCBCT_HIP(dev_malloc((void**)&d_tab, tab.size() * sizeof(double)));
     VCBCT_HIP(hipMemcpyAsync(d_tab, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    int zb = 4;
-    {
-        char key[128];
-        snprintf(key, sizeof key, "bp R%d Z%d n%d H%d W%d", R, Z, n, H, W);
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        auto it = g_bp_zb.find(key);
-        if (it != g_bp_zb.end()) zb = it->second;
-    }
-    int rc = launch_bp(zb, R, Z, zstart, step, scale, dev_recon, H, W, n, dev_sino, d_tab, xfactor, pitch_iso, st);
+    int rc = launch_bp(4, R, Z, zstart, step, scale, dev_recon, H, W, n, dev_sino, d_tab, xfactor, pitch_iso, st,
+                       bp_staged_fits(R, Z, step, scale, W, pitch_iso));
     (void)hipStreamSynchronize(st);
     (void)hipFree(d_tab);
     return rc;
@@ -1114,7 +1109,8 @@ extern "C" int vcbct_reconstruct_image_noalloc(int R, int Z, int zstart, double 
     hipLaunchKernelGGL(k_bp_table, dim3((n + 255) / 256), dim3(256), 0, st, dev_angles, dev_xshift, n, W, tab);
     VCBCT_HIP(hipGetLastError());
     // four slices per thread (the kernels give the same sums for every slice count)
-    return launch_bp(4, R, Z, zstart, step, scale, dev_recon, H, W, n, dev_sino, tab, xfactor, pitch_iso, st);
+    return launch_bp(4, R, Z, zstart, step, scale, dev_recon, H, W, n, dev_sino, tab, xfactor, pitch_iso, st,
+                     bp_staged_fits(R, Z, step, scale, W, pitch_iso));
 }
 
 extern "C" int vcbct_filter_sinogram_host(int H, int W, int n, const float* hp, float* ho, const double* xs,
