@@ -135,6 +135,17 @@ using namespace vcbct;
 
 static void free_multi(vcbct_projector* p);
 
+// Appends the sums that a ray which charges nothing needs (every exponential 1) to the spectrum pd of NE bins, in the
+// kernels' order: sum_e pdf_e, then sum_e pdf_e ch_ke for every channel k.
+constexpr int PDF_SUMS = 1 + VCBCT_MAX_MAT;
+static void pdf_sums(std::vector<double>& pd, const std::vector<double>& ch, int nch) {
+    const int NE = (int)pd.size();
+    pd.resize(NE + PDF_SUMS, 0.0);
+    for (int e = 0; e < NE; ++e) pd[NE] += pd[e];
+    for (int k = 0; k < nch; ++k)
+        for (int e = 0; e < NE; ++e) pd[NE + 1 + k] += pd[e] * ch[(size_t)k * NE + e];
+}
+
 extern "C" const char* vcbct_last_error(void) { return g_err; }
 
 extern "C" const char* vcbct_version(void) { return "vcbct 0.1 (gfx950)"; }
@@ -287,6 +298,8 @@ extern "C" int vcbct_projector_set_spectrum(vcbct_projector* p, const float* att
     std::vector<double> mu((size_t)nm * NE), pd(NE);
     for (size_t i = 0; i < mu.size(); ++i) mu[i] = atten[i];
     for (int e = 0; e < NE; ++e) pd[e] = pdf[e];
+    const std::vector<double>* chan = &mu;  // the adjoint's channel table
+    std::vector<double> ch;
     if (NE != p->NE) {
         (void)hipFree(p->d_mu);
         (void)hipFree(p->d_pdf);
@@ -298,13 +311,12 @@ extern "C" int vcbct_projector_set_spectrum(vcbct_projector* p, const float* att
         p->d_pdff = nullptr;
         p->NE = 0;
         if (dev_malloc((void**)&p->d_mu, mu.size() * sizeof(double)) != hipSuccess ||
-            dev_malloc((void**)&p->d_pdf, pd.size() * sizeof(double)) != hipSuccess ||
+            dev_malloc((void**)&p->d_pdf, (NE + PDF_SUMS) * sizeof(double)) != hipSuccess ||
             dev_malloc((void**)&p->d_muf, mu.size() * sizeof(float)) != hipSuccess ||
             dev_malloc((void**)&p->d_pdff, pd.size() * sizeof(float)) != hipSuccess)
             return fail(VCBCT_ENOMEM, "device allocation of the spectrum failed");
     }
     VCBCT_HIP(hipMemcpy(p->d_mu, mu.data(), mu.size() * sizeof(double), hipMemcpyHostToDevice));
-    VCBCT_HIP(hipMemcpy(p->d_pdf, pd.data(), pd.size() * sizeof(double), hipMemcpyHostToDevice));
     VCBCT_HIP(hipMemcpy(p->d_muf, atten, mu.size() * sizeof(float), hipMemcpyHostToDevice));
     VCBCT_HIP(hipMemcpy(p->d_pdff, pdf, pd.size() * sizeof(float), hipMemcpyHostToDevice));
     // The adjoint's channels.  When the table has a lower-rank form (mu = B (B^T mu) to 1e-6 of its largest
@@ -324,7 +336,8 @@ extern "C" int vcbct_projector_set_spectrum(vcbct_projector* p, const float* att
     p->chv_key = 0;
     p->fwd_ch = 0;
     if (r < nm) {
-        std::vector<double> ch((size_t)r * NE);
+        ch.resize((size_t)r * NE);
+        chan = &ch;
         std::vector<float> chf((size_t)r * NE);
         for (int k = 0; k < r; ++k)
             for (int e = 0; e < NE; ++e) {
@@ -339,6 +352,8 @@ extern "C" int vcbct_projector_set_spectrum(vcbct_projector* p, const float* att
         VCBCT_HIP(hipMemcpy(p->d_ch, ch.data(), ch.size() * sizeof(double), hipMemcpyHostToDevice));
         VCBCT_HIP(hipMemcpy(p->d_chf, chf.data(), chf.size() * sizeof(float), hipMemcpyHostToDevice));
     }
+    pdf_sums(pd, *chan, p->mix.nch);
+    VCBCT_HIP(hipMemcpy(p->d_pdf, pd.data(), pd.size() * sizeof(double), hipMemcpyHostToDevice));
     // The forward and the coefficient kernels traverse the channel volume (2 or 4 FP32 channels per voxel in
     // place of 6 u16 or 6 FP32 maps) when there are at most 4 channels and the basis keeps every bin's
     // exponent to ~1e-6 of itself; without a basis the channels are the maps themselves (nmat <= 4).
@@ -413,7 +428,7 @@ extern "C" int vcbct_projector_set_spectra(vcbct_projector* p, int nspec, const 
             }
         auto& t = p->ms[s];
         if (dev_malloc((void**)&t.d_mu, mu.size() * sizeof(double)) != hipSuccess ||
-            dev_malloc((void**)&t.d_pdf, pdd.size() * sizeof(double)) != hipSuccess ||
+            dev_malloc((void**)&t.d_pdf, (ne + PDF_SUMS) * sizeof(double)) != hipSuccess ||
             dev_malloc((void**)&t.d_muf, mu.size() * sizeof(float)) != hipSuccess ||
             dev_malloc((void**)&t.d_ch, ch.size() * sizeof(double)) != hipSuccess ||
             dev_malloc((void**)&t.d_chf, chf.size() * sizeof(float)) != hipSuccess) {
@@ -421,6 +436,7 @@ extern "C" int vcbct_projector_set_spectra(vcbct_projector* p, int nspec, const 
             return fail(VCBCT_ENOMEM, "device allocation of the spectra failed");
         }
         VCBCT_HIP(hipMemcpy(t.d_mu, mu.data(), mu.size() * sizeof(double), hipMemcpyHostToDevice));
+        pdf_sums(pdd, ch, nch);
         VCBCT_HIP(hipMemcpy(t.d_pdf, pdd.data(), pdd.size() * sizeof(double), hipMemcpyHostToDevice));
         VCBCT_HIP(hipMemcpy(t.d_muf, at, mu.size() * sizeof(float), hipMemcpyHostToDevice));
         VCBCT_HIP(hipMemcpy(t.d_ch, ch.data(), ch.size() * sizeof(double), hipMemcpyHostToDevice));

@@ -631,6 +631,10 @@ __device__ __forceinline__ double mubar_opaque(const float (&L)[VCBCT_MAX_MAT], 
     return xmin - log(se / sw);
 }
 
+// 2^x as the hardware gives it: exp2f without its steps for results below 2^-126, which come out as zero here.  (Such
+// terms are 1e-8 of the smallest sum that is not re-formed in FP64.)
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
 __device__ __forceinline__ bool all_zero(const float (&L)[VCBCT_MAX_MAT]) {
     bool z = true;
 #pragma unroll
@@ -751,37 +755,36 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
         if (zero) {
             for (int e = 0; e < NE; ++e) s += (float)(ldk(pdf, e) * 1.0 * leng);
         } else {
-            const float lf = (float)leng;
             const float k2 = (float)(-inv_xf * 1.4426950408889634);
+            float Lk[VCBCT_MAX_MAT];
+#pragma unroll
+            for (int m = 0; m < VCBCT_MAX_MAT; ++m) Lk[m] = L[m] * k2;
 #pragma unroll 4
             for (int e = 0; e < NE; ++e) {
                 float tr = 0.0f;
 #pragma unroll
                 for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
-                s += ldk(pdff, e) * exp2f(tr * k2) * lf;
+                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), Lk[m], tr);
+                s = fmaf(ldk(pdff, e), exp2_fast(tr), s);
             }
+            s *= (float)leng;
             // opaque ray: the FP32 exponentials underflow; the reference's own FP64 terms instead
             if (s < 1e-30f) s = intensity_exact(L, nl, mu, pdf, NE, inv_xf, leng);
         }
         stg(out, o, s);
     } else {  // VCBCT_MODE_LOGPROJ: p = -log(sum_e pdf_e e^{-mu.L/xf} / sum_e pdf_e); FP32 terms, FP64 sums
-        double sw = 0.0, se = 0.0;
+        const double sw = ldk(pdf, NE);
+        double se = sw;  // rays that charge nothing: every exponential is 1
         const float k2 = (float)(-inv_xf * 1.4426950408889634);
-        if (!__any(!zero)) {  // rays that charge nothing: every exponential is 1
-#pragma unroll 4
-            for (int e = 0; e < NE; ++e) sw += ldk(pdf, e);
-            se = sw;
-        } else {
+        if (__any(!zero)) {
+            se = 0.0;
 #pragma unroll 4
             for (int e = 0; e < NE; ++e) {
                 float tr = 0.0f;
 #pragma unroll
                 for (int m = 0; m < VCBCT_MAX_MAT; ++m)
                     if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
-                const double pe = ldk(pdf, e);
-                sw += pe;
-                se += pe * (double)exp2f(tr * k2);
+                se += ldk(pdf, e) * (double)exp2_fast(tr * k2);
             }
         }
         // opaque ray (the FP32 exponentials underflow): FP64 terms relative to the smallest exponent
@@ -997,7 +1000,8 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
     double lossc = 0.0;
     if (active) {
         // the exponent and its exponential in FP32 (relative error ~1e-6 per term), the sums in FP64
-        double sw = 0.0, se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
+        const double sw = ldk(pdf, NE);
+        double se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
         const float k2 = (float)(-inv_xf * 1.4426950408889634);
         if (__any(!all_zero(L))) {
 #pragma unroll 4
@@ -1006,24 +1010,17 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
 #pragma unroll
                 for (int m = 0; m < VCBCT_MAX_MAT; ++m)
                     if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
-                const double pe = ldk(pdf, e);
-                const double we = pe * (double)exp2f(tr * k2);
-                sw += pe;
+                const double we = ldk(pdf, e) * (double)exp2_fast(tr * k2);
                 se += we;
 #pragma unroll
                 for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nch) mub[m] += we * ldk(ch, m * NE + e);
+                    if (m < nch) mub[m] = fma(we, ldk(ch, m * NE + e), mub[m]);
             }
         } else {  // rays that charge nothing: every exponential is 1
-#pragma unroll 4
-            for (int e = 0; e < NE; ++e) {
-                const double pe = ldk(pdf, e);
-                sw += pe;
-#pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nch) mub[m] += pe * ldk(ch, m * NE + e);
-            }
             se = sw;
+#pragma unroll
+            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                if (m < nch) mub[m] = ldk(pdf, NE + 1 + m);
         }
         const size_t nrays = (size_t)g.nAng * g.H * g.W;
         const size_t o = (size_t)a * g.H * g.W + (size_t)(g.H - 1 - j) * g.W + jj;
@@ -1100,7 +1097,8 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(
             const double* __restrict__ pdf = ss.pdf[s];
             const float* __restrict__ muf = CHV ? ss.chf[s] : ss.muf[s];
             const double* __restrict__ ch = ss.ch[s];
-            double sw = 0.0, se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
+            const double sw = ldk(pdf, NE);
+            double se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
             if (charges) {
 #pragma unroll 4
                 for (int e = 0; e < NE; ++e) {
@@ -1108,22 +1106,15 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(
 #pragma unroll
                     for (int m = 0; m < VCBCT_MAX_MAT; ++m)
                         if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
-                    const double pe = ldk(pdf, e);
-                    const double we = pe * (double)exp2f(tr * k2);
-                    sw += pe;
+                    const double we = ldk(pdf, e) * (double)exp2_fast(tr * k2);
                     se += we;
 #pragma unroll
-                    for (int m = 0; m < NCH; ++m) mub[m] += we * ldk(ch, m * NE + e);
+                    for (int m = 0; m < NCH; ++m) mub[m] = fma(we, ldk(ch, m * NE + e), mub[m]);
                 }
             } else {  // rays that charge nothing: every exponential is 1
-#pragma unroll 4
-                for (int e = 0; e < NE; ++e) {
-                    const double pe = ldk(pdf, e);
-                    sw += pe;
-#pragma unroll
-                    for (int m = 0; m < NCH; ++m) mub[m] += pe * ldk(ch, m * NE + e);
-                }
                 se = sw;
+#pragma unroll
+                for (int m = 0; m < NCH; ++m) mub[m] = ldk(pdf, NE + 1 + m);
             }
             double p;
             if (se < 1e-30 * sw) {  // opaque ray: FP64 terms relative to the smallest exponent
@@ -1172,7 +1163,8 @@ __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const fl
         float L[VCBCT_MAX_MAT];
 #pragma unroll
         for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = m < nl ? ldg(Ls, (size_t)m * nrays + o) : 0.0f;
-        double sw = 0.0, se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
+        const double sw = ldk(pdf, NE);
+        double se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
         const float k2 = (float)(-inv_xf * 1.4426950408889634);
         if (__any(!all_zero(L))) {
 #pragma unroll 4
@@ -1181,24 +1173,17 @@ __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const fl
 #pragma unroll
                 for (int m = 0; m < VCBCT_MAX_MAT; ++m)
                     if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
-                const double pe = ldk(pdf, e);
-                const double we = pe * (double)exp2f(tr * k2);
-                sw += pe;
+                const double we = ldk(pdf, e) * (double)exp2_fast(tr * k2);
                 se += we;
 #pragma unroll
                 for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nch) mub[m] += we * ldk(ch, m * NE + e);
+                    if (m < nch) mub[m] = fma(we, ldk(ch, m * NE + e), mub[m]);
             }
         } else {  // rays that charge nothing: every exponential is 1
-#pragma unroll 4
-            for (int e = 0; e < NE; ++e) {
-                const double pe = ldk(pdf, e);
-                sw += pe;
-#pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nch) mub[m] += pe * ldk(ch, m * NE + e);
-            }
             se = sw;
+#pragma unroll
+            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                if (m < nch) mub[m] = ldk(pdf, NE + 1 + m);
         }
         if (se < 1e-30 * sw) {  // opaque ray: FP64 terms relative to the smallest exponent
             (void)mubar_opaque(L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, nch);

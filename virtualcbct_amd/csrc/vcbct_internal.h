@@ -86,7 +86,7 @@ __device__ __forceinline__ void stg(T* p, size_t i, T v) {
 // Per-call spectrum view (device pointers to FP64 copies of the reference's float tables).
 struct Spectrum {
     const double* mu;   // [nmat][NE]
-    const double* pdf;  // [NE]
+    const double* pdf;  // [NE], then its sum and, per channel k, sum_e pdf_e ch_ke (read by the adjoint and log projection)
     const float* muf;   // the same tables as given (FP32): the intensity projection's spectral sum
     const float* pdff;
     int NE;
@@ -111,7 +111,7 @@ enum VoxKind { VOX_U16 = 0, VOX_F32 = 1, VOX_CH2 = 2, VOX_CH4 = 3 };
 #define VCBCT_MAX_SPECTRA 4
 struct SpecSet {
     const double* mu[VCBCT_MAX_SPECTRA];   // [nmat][NE_s]
-    const double* pdf[VCBCT_MAX_SPECTRA];  // [NE_s]
+    const double* pdf[VCBCT_MAX_SPECTRA];  // [NE_s], then the sums as in Spectrum
     const float* muf[VCBCT_MAX_SPECTRA];   // [nmat][NE_s] as given
     const double* ch[VCBCT_MAX_SPECTRA];   // [nch][NE_s], the channel table of spectrum s
     const float* chf[VCBCT_MAX_SPECTRA];   // the same in FP32
