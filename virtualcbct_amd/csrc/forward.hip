@@ -453,6 +453,14 @@ template <bool ORDERED, class VoxT>
 __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double sn, double xc, double yc, int j, int jj,
                                            bool active, const VoxT* __restrict__ vox, float (&L)[VCBCT_MAX_MAT],
                                            WalkLds* lds) {
+    {
+        const int jw = __builtin_amdgcn_readfirstlane(j - (int)(threadIdx.x & 63));  // the wave's first row
+        if (rows_miss(g, yc, jw, jw + 63 < g.H ? jw + 63 : g.H - 1)) {
+#pragma unroll
+            for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = 0.0f;
+            return ray_leng(g, xc, yc, active ? j : 0, jj);
+        }
+    }
     RayCtx r;
     ray_setup(g, c, sn, xc, yc, active ? j : 0, jj, r);
     share_xy_path(r);

@@ -38,6 +38,7 @@ struct ProjGeom {
     double rmax2;           // squared radius of the inscribed-circle mask, (N/2 * s)^2
     int aligned;            // 1/s integral: the whole-cm plane grid lies on voxel boundaries
     int mul24;              // N * Nz < 2^24: voxel strides multiply in 24 bits
+    double lam0, lam1;      // bounds of the volume's points as fractions of the way from the source to the panel; 0: none
 };
 
 // Fills the derived fields of a ProjGeom whose primary fields are set.
@@ -53,6 +54,12 @@ inline void derive_geom(ProjGeom& g) {
     const double q = 1.0 / g.s;
     g.aligned = (q >= 1.0 && std::fabs(q - std::rint(q)) < 1e-9) ? 1 : 0;
     g.mul24 = ((long long)g.N * g.Nz < (1LL << 24)) ? 1 : 0;
+    // a point of the volume lies within `a` of the axis, the panel's plane within `a` too (registration shifts)
+    const double a = 1.4143 * (g.lim_u + g.s) + 2.0 * (std::fabs(g.x_reg) + std::fabs(g.y_reg)) *
+                                                    std::fmax(1.0, g.pitch_iso / g.pitch);
+    const bool bounded = a < 0.4 * g.sad;
+    g.lam0 = bounded ? (g.sad - a) / (g.sad + a) : 0.0;
+    g.lam1 = bounded ? (g.sad + a) / (g.sad - a) : 0.0;
 }
 
 #ifdef __HIPCC__
