@@ -25,10 +25,11 @@ constexpr int SZ = 32;  // slices of a tile: 64 KB of FP64 sums a channel; a CU'
 constexpr int SK = 20;  // steps of a ray in a tile: at most ST + 1 voxels along the major axis, and one each side
 
 // The xy path of the rays of one detector column at one angle (the same for all its rows), made by k_scatter_rays.
-// iM = 1 / (pu - su), q1 = 1 + dv^2; entry: the voxel column (y << 16 | x) of the lumped entry segment, or -1.
+// iM = 1 / (pu - su), q1 = 1 + dv^2, M = |pu - su|; entry: the voxel column (y << 16 | x) of the lumped entry segment, or -1.
 struct alignas(16) ScatterRay {
     double su, sv, dv, duv, ui, uin, iM, q1;
-    int flags, nb, entry, pad;
+    int flags, nb, entry;
+    float M;
 };
 enum { SR_LIVE = 1, SR_XMAJ = 2, SR_VMOVE = 4, SR_PHA = 8, SR_DIRV = 16 };
 
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(256) void k_scatter_rays(ProjGeom g, const double* 
     o.uin = r.uin;
     o.iM = 1.0 / (r.pu - r.su);
     o.q1 = 1.0 + r.dv * r.dv;
-    o.pad = 0;
+    o.M = (float)fabs(r.pu - r.su);
     o.entry = -1;
     o.flags = 0;
     o.nb = 0;
@@ -150,8 +151,9 @@ __global__ __launch_bounds__(512 * NCH) __attribute__((amdgpu_waves_per_eu(4, 4)
     const size_t nrays = (size_t)g.nAng * g.H * g.W;
     const double pixh = g.pitch_iso * (g.pixnum / g.H), ipixh = 1.0 / pixh;
     const double zreg = g.z_reg * g.pitch_iso / g.pitch;
-    // the chunk's z range (slice 0 also takes the truncated range above it)
-    const double zl = (double)(nzm - zc - nz) * g.t, zh = (double)(nzm - zc + (zc == 0 ? 1 : 0)) * g.t;
+    // the chunk's z range relative to the source's (slice 0 also takes the truncated range above it)
+    const float zlf = (float)((double)(nzm - zc - nz) * g.t - g.z_reg);
+    const float zhf = (float)((double)(nzm - zc + (zc == 0 ? 1 : 0)) * g.t - g.z_reg);
 
     for (;;) {
         int task = 0;
@@ -244,13 +246,14 @@ __global__ __launch_bounds__(512 * NCH) __attribute__((amdgpu_waves_per_eu(4, 4)
                             : -1;
                 // the rows whose rays can be in the chunk's slices within these steps
                 const double D0 = (plane_u(r, k0 - 1, g.s) - r.su) * r.pha;
-                const double Da = ecell >= 0 ? fmin(D0, (R.ui - r.su) * r.pha) : D0;
-                const double Db = D0 + (nsteps + 1) * g.s, M = fabs(1.0 / R.iM);
-                const double qa = M / Da, qb = M / Db;
-                const double pl = (zl - g.z_reg) * (zl > g.z_reg ? qb : qa) + g.z_reg;
-                const double ph = (zh - g.z_reg) * (zh > g.z_reg ? qa : qb) + g.z_reg;
-                j0 = (int)fmin(fmax(floor((zreg - ph) * ipixh - yc - 0.01), 0.0), (double)g.H);
-                j1 = (int)fmax(fmin(ceil((zreg - pl) * ipixh - yc + 0.01), (double)(g.H - 1)), -1.0);
+                // (FP32: off by less than the hundredth of a row that is added on either side)
+                const float Da = (float)(ecell >= 0 ? fmin(D0, (R.ui - r.su) * r.pha) : D0);
+                const float Db = (float)(D0 + (nsteps + 1) * g.s);
+                const float qa = R.M * __builtin_amdgcn_rcpf(Da), qb = R.M * __builtin_amdgcn_rcpf(Db);
+                const float pl = zlf * (zlf > 0.0f ? qb : qa), ph = zhf * (zhf > 0.0f ? qa : qb);  // pz - sz
+                const float row0 = (float)((zreg - g.z_reg) * ipixh - yc), ip = (float)ipixh;
+                j0 = (int)fminf(fmaxf(floorf(row0 - ph * ip - 0.02f), 0.0f), (float)g.H);
+                j1 = (int)fmaxf(fminf(ceilf(row0 - pl * ip + 0.02f), (float)(g.H - 1)), -1.0f);
                 // (a part of a piece that the tile does not list can have its own midpoint in the tile, or in the circle)
                 if (!(total > 0 || parts || ecell >= 0)) j1 = j0 - 1;
                 __builtin_amdgcn_wave_barrier();
@@ -297,10 +300,11 @@ __global__ __launch_bounds__(512 * NCH) __attribute__((amdgpu_waves_per_eu(4, 4)
                     if (!__any(any)) continue;
                     const double pz = -(yc + j) * g.pitch_iso * (g.pixnum / g.H) + zreg;
                     r.dz = (pz - r.sz) * iM;
-                    {  // the length per unit of u: sqrt in FP32 and one Newton step in FP64
+                    {  // the length per unit of u: the root in FP32 and one Newton step in FP64
                         const double qq = q1 + r.dz * r.dz;
-                        const float k = sqrtf((float)qq);
-                        const double K = (double)k + (qq - (double)k * k) * (double)(0.5f / k);
+                        const float h = __builtin_amdgcn_rsqf((float)qq);
+                        const double k = (double)((float)qq * h);
+                        const double K = k + (qq - k * k) * (double)(0.5f * h);
 #pragma unroll
                         for (int m = 0; m < NCH; ++m) cm[m] *= K;
                     }
@@ -336,18 +340,23 @@ __global__ __launch_bounds__(512 * NCH) __attribute__((amdgpu_waves_per_eu(4, 4)
                     if (ce >= 0 && on) segment(ldk(&RP->ui, 0), r.uin, ce);
                     // the lane's slice and next slice plane at the first step (as walk_runs)
                     const double fA = r.pha * r.dz * c.ninv_t;
-                    const double duzD = r.pha / r.dz;
+                    // pha / dz, a rounding off at most (dz = 0: not used)
+                    double duzD = __builtin_amdgcn_rcp(r.dz);
+                    duzD = fma(fma(-r.dz, duzD, 1.0), duzD, duzD);
+                    duzD = fma(fma(-r.dz, duzD, 1.0), duzD, duzD) * r.pha;
                     const int up = fA > 0.0 ? 1 : 0, sgn = fA > 0.0 ? 1 : -1;
                     auto plane_at = [&](int mm) -> double {
                         const int p = nzm - mm;
                         const double zb = p * sgn > 0 ? (double)(p - sgn) * g.t + (double)sgn * g.t : (double)p * g.t;
                         return on && fA != 0.0 ? (zb - r.sz) * duzD : 1.0e300;
                     };
-                    int il = (int)fmin(fmax(floor((D0 + 1e-3 * g.s) * fA + (r.sz * c.ninv_t + c.nzm)), -1.0e9), 1.0e9);
+                    const double fB = r.sz * c.ninv_t + c.nzm;
+                    int il = (int)floor((D0 + 1e-3 * g.s) * fA + fB);  // (saturates far outside the volume)
                     double dnext = plane_at(il + up);
-                    if (on && fA != 0.0) {
+                    // (a plane within the first thousandth of the first step is met in that step)
+                    if (__any(on && (int)floor(D0 * fA + fB) != il)) {
                         const double Dprev = plane_at(il + up - sgn);
-                        if (Dprev > D0) {
+                        if (on && fA != 0.0 && Dprev > D0) {
                             il -= sgn;
                             dnext = Dprev;
                         }
@@ -372,15 +381,19 @@ __global__ __launch_bounds__(512 * NCH) __attribute__((amdgpu_waves_per_eu(4, 4)
                             int kc = (int)((dnext - D0) * g.inv_s);
                             kc = kc < kb ? kb : (kc >= ke ? ke - 1 : kc);
                             const int fl = S->flags[kc];
-                            const double Db0 = pos_of(ck0 + kc - 1), Dk = pos_of(ck0 + kc), Dv = r.pha * S->dv[kc];
+                            const double Dk = pos_of(ck0 + kc), Dv = r.pha * S->dv[kc];
                             const bool splitv = (fl & STEP_SPLITV) != 0;
                             const bool tie = splitv && fabs(Dk - dnext) == fabs(Dk - Dv);
                             const bool z0 = !splitv || dnext < Dv;
-                            const double ba = z0 ? Db0 : Dv, be = z0 && splitv ? Dv : Dk;
+                            const double be = z0 && splitv ? Dv : Dk;
                             const bool listed = (fl & (z0 ? STEP_OK0 : STEP_OK1)) != 0;
                             const bool zero = il + up == nzm;  // the z = 0 plane splits nothing: whole, by the midpoint
                             const bool special = !zero && ((fl & RUN_SPECIAL) || tie);
-                            const double at = zero ? ((ba + be) * 0.5 < dnext ? be : ba) : dnext;
+                            double at = dnext;
+                            if (__any(zero)) {
+                                const double ba = z0 ? pos_of(ck0 + kc - 1) : Dv;
+                                if (zero) at = (ba + be) * 0.5 < dnext ? be : ba;
+                            }
                             px = (fl >> RUN_SHIFT) + (!z0 && (fl & STEP_OK0) ? 1 : 0);
                             first_new = px + (listed ? 1 : 0);
                             moved = listed;
