@@ -723,6 +723,7 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
                                              const float* __restrict__ pdff, int NE, double inv_xf, int nl, int a,
                                              int rg, int jj, float* __restrict__ out, float* __restrict__ aux,
                                              WalkLds* steps) {
+    constexpr int NT = RunRec<VoxT>::kTerms;  // bound of nl
     const int lane = threadIdx.x & 63;
     const int j = rg * 64 + lane;
     const bool active = j < g.H;
@@ -771,7 +772,7 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
             for (int e = 0; e < NE; ++e) {
                 float tr = 0.0f;
 #pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                for (int m = 0; m < NT; ++m)
                     if (m < nl) tr = fmaf(ldk(muf, m * NE + e), Lk[m], tr);
                 s = fmaf(ldk(pdff, e), exp2_fast(tr), s);
             }
@@ -790,7 +791,7 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
             for (int e = 0; e < NE; ++e) {
                 float tr = 0.0f;
 #pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                for (int m = 0; m < NT; ++m)
                     if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
                 se += ldk(pdf, e) * (double)exp2_fast(tr * k2);
             }
@@ -993,6 +994,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
                                                       float* __restrict__ coef, double* __restrict__ loss) {
     __shared__ WalkLds step_tabs[4];
     WalkLds* steps = &step_tabs[threadIdx.x >> 6];
+    constexpr int NT = RunRec<VoxT>::kTerms;  // bound of nl and nch
     const Tile t = tile_map(tm, g.nAng);
     const int lane = threadIdx.x & 63;
     const int j = t.rg * 64 + lane;
@@ -1016,18 +1018,18 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
             for (int e = 0; e < NE; ++e) {
                 float tr = 0.0f;
 #pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                for (int m = 0; m < NT; ++m)
                     if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
                 const double we = ldk(pdf, e) * (double)exp2_fast(tr * k2);
                 se += we;
 #pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                for (int m = 0; m < NT; ++m)
                     if (m < nch) mub[m] = fma(we, ldk(ch, m * NE + e), mub[m]);
             }
         } else {  // rays that charge nothing: every exponential is 1
             se = sw;
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+            for (int m = 0; m < NT; ++m)
                 if (m < nch) mub[m] = ldk(pdf, NE + 1 + m);
         }
         const size_t nrays = (size_t)g.nAng * g.H * g.W;
@@ -1038,7 +1040,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
         } else {
             p = -log(se / sw);
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m) mub[m] /= se;
+            for (int m = 0; m < NT; ++m) mub[m] /= se;
         }
         double w;
         if (MODE == VCBCT_ADJ_LOSS) {
@@ -1049,7 +1051,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
             w = (double)ldg(tg, o);
         }
 #pragma unroll
-        for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+        for (int m = 0; m < NT; ++m)
             if (m < nch) stg(coef, (size_t)m * nrays + ((size_t)a * g.W + jj) * g.H + j, (float)(w * mub[m] * inv_xf));
     }
     if (MODE == VCBCT_ADJ_LOSS && loss) {
@@ -1112,7 +1114,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(
                 for (int e = 0; e < NE; ++e) {
                     float tr = 0.0f;
 #pragma unroll
-                    for (int m = 0; m < VCBCT_MAX_MAT; ++m)
+                    for (int m = 0; m < (CHV ? NCH : VCBCT_MAX_MAT); ++m)
                         if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
                     const double we = ldk(pdf, e) * (double)exp2_fast(tr * k2);
                     se += we;
@@ -1150,9 +1152,11 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(
 }
 
 // The coefficients of the upstream-gradient mode from line integrals saved by the forward log projection
-// (the same traversal, so the same FP32 sums): one thread per ray, the epilogue of k_adjoint_coef.  A block takes 16 x 16
-// rays of an angle, so that the reads (along the detector row) and the writes (along the column) both keep to
-// 64-byte runs.
+// (the same traversal, so the same FP32 sums): the epilogue of k_adjoint_coef.  A block takes 32 x 32 rays of an angle, four
+// rows of 32 columns a pass, and turns the coefficients in LDS: the reads run along the detector row, the writes along the
+// column, both in 128-byte lines.  (With 16 x 16 rays and no LDS, 64-byte reads and 16-byte writes a wave: 57.6e6 rays of
+// one channel took 467 us, 247 so.)  NT: bound of nl and nch.
+template <int NT>
 __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const float* __restrict__ Ls,
                                                             const double* __restrict__ mu,
                                                             const double* __restrict__ pdf,
@@ -1160,49 +1164,64 @@ __global__ __launch_bounds__(256) void k_adjoint_coef_saved(ProjGeom g, const fl
                                                             const double* __restrict__ ch, int nch, int NE,
                                                             double inv_xf, int nl, const float* __restrict__ gp,
                                                             float* __restrict__ coef) {
+    __shared__ float tile[NT][32][33];
     const size_t nrays = (size_t)g.nAng * g.H * g.W;
-    const int ncb = (g.W + 15) / 16, nrb = (g.H + 15) / 16;
+    const int ncb = (g.W + 31) / 32, nrb = (g.H + 31) / 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const double sw = ldk(pdf, NE);
+    const float k2 = (float)(-inv_xf * 1.4426950408889634);
     for (size_t b = blockIdx.x; b < (size_t)g.nAng * ncb * nrb; b += gridDim.x) {
         const int a = (int)(b / ((size_t)ncb * nrb)), rc = (int)(b % ((size_t)ncb * nrb));
-        const int jj = rc % ncb * 16 + (threadIdx.x & 15), row = rc / ncb * 16 + (threadIdx.x >> 4);
-        if (jj >= g.W || row >= g.H) continue;
-        const size_t o = ((size_t)a * g.H + row) * g.W + jj;
-        const size_t oc = ((size_t)a * g.W + jj) * g.H + (g.H - 1 - row);
-        float L[VCBCT_MAX_MAT];
+        const int col0 = rc % ncb * 32, row0 = rc / ncb * 32;
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i) {
+            const int jj = col0 + tx, row = row0 + ty + 8 * i;
+            if (jj >= g.W || row >= g.H) continue;
+            const size_t o = ((size_t)a * g.H + row) * g.W + jj;
+            float L[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = m < nl ? ldg(Ls, (size_t)m * nrays + o) : 0.0f;
-        const double sw = ldk(pdf, NE);
-        double se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
-        const float k2 = (float)(-inv_xf * 1.4426950408889634);
-        if (__any(!all_zero(L))) {
+            for (int m = 0; m < NT; ++m) L[m] = m < nl ? ldg(Ls, (size_t)m * nrays + o) : 0.0f;
+            const double w = (double)ldg(gp, o);
+            double se = 0.0, mub[VCBCT_MAX_MAT] = {0, 0, 0, 0, 0, 0};
+            if (__any(!all_zero(L))) {
 #pragma unroll 4
-            for (int e = 0; e < NE; ++e) {
-                float tr = 0.0f;
+                for (int e = 0; e < NE; ++e) {
+                    float tr = 0.0f;
 #pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
-                const double we = ldk(pdf, e) * (double)exp2_fast(tr * k2);
-                se += we;
+                    for (int m = 0; m < NT; ++m)
+                        if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
+                    const double we = ldk(pdf, e) * (double)exp2_fast(tr * k2);
+                    se += we;
 #pragma unroll
-                for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                    if (m < nch) mub[m] = fma(we, ldk(ch, m * NE + e), mub[m]);
+                    for (int m = 0; m < NT; ++m)
+                        if (m < nch) mub[m] = fma(we, ldk(ch, m * NE + e), mub[m]);
+                }
+            } else {  // rays that charge nothing: every exponential is 1
+                se = sw;
+#pragma unroll
+                for (int m = 0; m < NT; ++m)
+                    if (m < nch) mub[m] = ldk(pdf, NE + 1 + m);
             }
-        } else {  // rays that charge nothing: every exponential is 1
-            se = sw;
+            if (se < 1e-30 * sw) {  // opaque ray: FP64 terms relative to the smallest exponent
+                (void)mubar_opaque(L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, nch);
+            } else {
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-                if (m < nch) mub[m] = ldk(pdf, NE + 1 + m);
+                for (int m = 0; m < NT; ++m) mub[m] /= se;
+            }
+#pragma unroll
+            for (int m = 0; m < NT; ++m)
+                if (m < nch) tile[m][tx][ty + 8 * i] = (float)(w * mub[m] * inv_xf);
         }
-        if (se < 1e-30 * sw) {  // opaque ray: FP64 terms relative to the smallest exponent
-            (void)mubar_opaque(L, nl, mu, pdf, NE, inv_xf, sw, mub, ch, nch);
-        } else {
+        __syncthreads();
+        for (int i = 0; i < 4; ++i) {
+            const int jj = col0 + ty + 8 * i, row = row0 + tx;
+            if (jj >= g.W || row >= g.H) continue;
+            const size_t oc = ((size_t)a * g.W + jj) * g.H + (g.H - 1 - row);
 #pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m) mub[m] /= se;
+            for (int m = 0; m < NT; ++m)
+                if (m < nch) stg(coef, (size_t)m * nrays + oc, tile[m][ty + 8 * i][tx]);
         }
-        const double w = (double)ldg(gp, o);
-#pragma unroll
-        for (int m = 0; m < VCBCT_MAX_MAT; ++m)
-            if (m < nch) stg(coef, (size_t)m * nrays + oc, (float)(w * mub[m] * inv_xf));
+        __syncthreads();
     }
 }
 
@@ -1717,10 +1736,16 @@ int launch_adjoint_multi(const ProjGeom& g, const double* tables, const void* vo
 int launch_adjoint_saved(const ProjGeom& g, const double* tables, const float* Ls, const Spectrum& sp,
                          double xfactor, const float* gp, float* coef, float* grad_vox, hipStream_t st,
                          const TileShape& forced) {
-    const unsigned nbc =
-        (unsigned)std::min<size_t>((size_t)g.nAng * ((g.H + 15) / 16) * ((g.W + 15) / 16), 65536);
-    hipLaunchKernelGGL(k_adjoint_coef_saved, dim3(nbc), dim3(256), 0, st, g, Ls, sp.mu, sp.pdf, sp.muf, sp.ch, sp.nch,
-                       sp.NE, 1.0 / xfactor, sp.nl, gp, coef);
+    const unsigned nbc = (unsigned)std::min<size_t>((size_t)g.nAng * ((g.H + 31) / 32) * ((g.W + 31) / 32), 65536);
+    const int nt = std::max(sp.nl, sp.nch);
+#define VCBCT_LAUNCH_SAVED(T)                                                                                        \
+    hipLaunchKernelGGL(k_adjoint_coef_saved<T>, dim3(nbc), dim3(256), 0, st, g, Ls, sp.mu, sp.pdf, sp.muf, sp.ch,    \
+                       sp.nch, sp.NE, 1.0 / xfactor, sp.nl, gp, coef)
+    if (nt <= 1) VCBCT_LAUNCH_SAVED(1);
+    else if (nt <= 2) VCBCT_LAUNCH_SAVED(2);
+    else if (nt <= 4) VCBCT_LAUNCH_SAVED(4);
+    else VCBCT_LAUNCH_SAVED(6);
+#undef VCBCT_LAUNCH_SAVED
     VCBCT_HIP(hipGetLastError());
     return run_scatter(g, tables, coef, sp.nch, grad_vox, st, forced);
 }
