@@ -704,8 +704,8 @@ __global__ __launch_bounds__(256) void k_backproject(float* __restrict__ recon, 
 // footprint is theirs, widened by more than a rounding.  An angle whose footprint leaves the panel, or the tile, goes
 // through the loads, clamps and selects of k_backproject.  Two sets of buffers alternate: one barrier per four angles.
 // k_backproject is bound by its taps in the vector L1 (~20 cycles per two-word load of a wave: 2.7 ms on 270x270x128 / 360
-// angles of 400x400); from LDS they are two paired reads, and the kernel is bound by vector issue (~17 instructions an
-// update, 11 of them the interpolation): 1.68 ms with 8 slices a thread, 1.77 with 4.
+// angles of 400x400); from LDS they are two paired reads, and the kernel is bound by vector issue (14 instructions an
+// update, 11 of them the interpolation) beside the LDS reads: 1.68 ms with 8 slices a thread, 1.77 with 4.
 // Eight slices a thread span up to 58 rows there, four 30.  The taller tile has one buffer (and a second barrier), so
 // that four blocks fit a CU's 160 KB either way.
 constexpr int BP_TC = 32;

@@ -17,8 +17,8 @@
 // the midpoint, and equal crossing distances charge the whole chord once.  Where those need a part's own midpoint
 // (a step at the circle's boundary, equal distances, a plane grid off the voxel grid) the parts are formed as the
 // step walk forms its segments.
-// What bounds it: on the 512x512x128 / 360-angle projection the gathers' traffic beyond L2 (~9e10 bytes at 8.5 TB/s);
-// the step walk took 20.7 ms there, bound by vector issue (1.19e10 wave-instructions), this walk 10.6 ms.
+// What bounds it: on the 512x512x128 / 360-angle projection the gathers' traffic beyond L2 (7.7e10 bytes at 7.4 TB/s);
+// the step walk took 20.7 ms there, bound by vector issue (1.19e10 wave-instructions, now 4.5e9), this walk 10.5 ms.
 // A piece's length is its extent along the major axis times the ray's length factor, multiplied per piece as the step
 // walk does: FP32 sums of equal terms (a constant map) round one way, and by the terms' own digits, so lengths scaled
 // once at the end would leave a log projection 1e-7 off the step walk's there.

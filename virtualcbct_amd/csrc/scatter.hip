@@ -6,9 +6,9 @@
 // dual-energy gradient of a 512x512x64 / 360-angle problem.  Here a block owns a tile of ST x ST voxel columns by SZ
 // slices in LDS, visits every ray that crosses the tile at the angles of its group, and adds the tile to the gradient
 // once at the end, so that a voxel costs one global atomic per angle group instead of one per ray.
-// Measured: that scatter 38.8 -> 14.1 ms, 256x256x64 / 360 angles / one channel 11.4 -> 2.9 ms, 256x256x64 / 90 angles of
-// 256x256 / two channels 2.87 -> 1.2 ms.  What bounds it now is vector issue (5.5e9 wave-instructions, 63 % of the
-// cycles; a fifth of them the steps of the columns, formed anew for every tile) beside the LDS atomics (50 %).
+// Measured: that scatter 38.8 -> 13.1 ms, 256x256x64 / 360 angles / one channel 11.4 -> 6.0 ms, 256x256x64 / 90 angles of
+// 256x256 / two channels 2.87 -> 1.2 ms.  What bounds it now is vector issue (4.8e9 wave-instructions, 60 % of the
+// cycles; a fifth of them the steps of the columns, formed anew for every tile) beside the LDS atomics (55 %).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -39,15 +39,16 @@ size_t scatter_work_bytes(const ProjGeom& g) {
     return scatter_ray_bytes(g) + 16 + (size_t)g.nAng * g.W * sizeof(int);
 }
 
-// The tile form's range: 15-bit voxel indices, and a source well outside the volume (the tile's footprint on the panel
-// is its corners' projection); and at least 4e7 ray steps, as a tile costs its clearing and its final atomics whatever
+// The tile form's range: 15-bit voxel indices, rows and columns (the latter formed in FP32 with margins of a fiftieth), a
+// slice chunk per grid layer, and a source well outside the volume (the tile's footprint on the panel is its corners'
+// projection); and at least 4e7 ray steps, as a tile costs its clearing and its final atomics whatever
 // it gathers.  Backward from saved line integrals, ray-ordered against tiles: 64x64x20 / 24 angles of 60x60 (5.5e6) 163
 // against 207 us over five channels, with 90 angles (2.1e7) 380 against 488, with 360 (8.3e7) 1272 against 1119;
 // 128x128x32 / 24 angles of 128x128 (5.0e7) 408 against 475, over two channels 256 against 217, over one 195 against 108;
 // 256x256x64 / 8 angles of 256x256 (1.3e8) 798 against 716 over five, 290 against 184 over one.
 bool scatter_by_tiles(const ProjGeom& g) {
     const double reach = (0.5 * g.N + 1.0) * g.s * 3.0 + std::fabs(g.x_reg) + std::fabs(g.y_reg);
-    return g.N < 32768 && reach < g.sad && (size_t)g.nAng * g.W < (size_t)INT_MAX &&
+    return g.N < 32768 && g.H < 32768 && g.W < 32768 && (g.Nz + SZ - 1) / SZ <= 65535 && reach < g.sad && (size_t)g.nAng * g.W < (size_t)INT_MAX &&
            (double)g.nAng * g.H * g.W * g.N >= 4.0e7;
 }
 
