@@ -32,10 +32,16 @@ namespace vcbct {
 // and 12.6 at 8 (where the scalar registers spill too); with the step walk it took 20.7 ms.  The ordered form needs
 // 4 (54.1 ms for the dual-energy gradient of a 512x512x64 / 360-angle problem; 54.6 at 5 with spills).
 #define VCBCT_WAVES8 __attribute__((amdgpu_waves_per_eu(8, 8)))
+// The projection kernels that hold the step walk alone (volumes past the run walk's reach, thin slices, segment counts)
+// are held to 7, the intensity to 8: 700x700x600 two-channel slices / 12 angles of 400x400, log projection 3.9 ms at 5
+// waves, 3.7 at 7.
 #define VCBCT_WAVES_RUN __attribute__((amdgpu_waves_per_eu(5, 5)))
-#define VCBCT_WAVES_ORDERED __attribute__((amdgpu_waves_per_eu(4, 4)))
-#define VCBCT_WAVES_COEF(MODE) \
-    __attribute__((amdgpu_waves_per_eu((MODE) == VCBCT_ADJ_LOSS ? 4 : 5, (MODE) == VCBCT_ADJ_LOSS ? 4 : 5)))
+#define VCBCT_WAVES_FWD(MODE, RUNS)               \
+    __attribute__((amdgpu_waves_per_eu((RUNS) ? 5 : (MODE) == VCBCT_MODE_INTENSITY ? 8 : 7, (RUNS) ? 5 : 8)))
+#define VCBCT_WAVES_COEF(MODE, RUNS)                                                                   \
+    __attribute__((amdgpu_waves_per_eu(!(RUNS) ? 8 : (MODE) == VCBCT_ADJ_LOSS ? 4 : 5,                  \
+                                       !(RUNS) ? 8 : (MODE) == VCBCT_ADJ_LOSS ? 4 : 5)))
+#define VCBCT_WAVES_MULTI(RUNS) __attribute__((amdgpu_waves_per_eu((RUNS) ? 4 : 7, (RUNS) ? 4 : 8)))
 
 // ------------------------------------------------------------------------------------------------
 // Volume re-layout.  Reference u16 [z][mat][y][x] -> device [y][x][z][8] (16-byte voxel, all materials;
@@ -446,10 +452,26 @@ struct OrderedAcc : RunAcc<VoxT> {
     }
 };
 
-// The line integrals of one wave's rays into L: by runs where the wave's lanes share their xy path, no lane can meet
-// two slice planes in one step and the volume is within the gathers' reach, else step by step.  ORDERED: bit for bit
-// the step walk's sums (plane grids off the voxel grid keep that walk).  Returns the lane's cos^3 factor.
-template <bool ORDERED, class VoxT>
+// Fewest steps a block of the run walk may hold for it to be taken.  With one, the step table is the faster: 128x128x533
+// slices of 0.12 mm / 48 angles of 128x128, log projection over two channels 477 us by runs against 321, off the plane
+// grid 644 against 499; with two and three, runs are (0.25 mm: 222 against 287 us).  The ordered walk needs four: 0.5 mm
+// slices there, loss gradient over two channels 1.72 ms in blocks of one step on, 1.32 of two on, 1.31 of four on, 1.26
+// by steps alone; 1 mm 0.88 / 0.88 / 0.81 / 0.80 ms; on 256x256x128 / 24 angles of 256x256 runs of four on win, 2.17
+// against 2.24 ms.
+template <bool ORDERED>
+constexpr int kRunSteps = ORDERED ? 4 : 2;
+
+// Whether waves of the geometry may take the run walk: the volume within the gathers' reach, slices not too thin.
+template <class VoxT>
+__host__ __device__ __forceinline__ bool run_walk(const ProjGeom& g) {
+    return (size_t)g.N * g.N * g.Nz <= (size_t)RunAcc<VoxT>::kOut && !g.thin;
+}
+
+// The line integrals of one wave's rays into L: by runs where the wave's lanes share their xy path, a block holds enough
+// steps (two slice planes in one step: none) and the volume is within the gathers' reach, else step by step.
+// ORDERED: bit for bit the step walk's sums (plane grids off the voxel grid keep that walk).  RUNS false: the step walk
+// alone (run_walk).  Returns the lane's cos^3 factor.
+template <bool ORDERED, bool RUNS, class VoxT>
 __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double sn, double xc, double yc, int j, int jj,
                                            bool active, const VoxT* __restrict__ vox, float (&L)[VCBCT_MAX_MAT],
                                            WalkLds* lds) {
@@ -472,14 +494,16 @@ __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double s
     for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = 0.0f;
     if (kmin > kmax) return r.leng;  // no lane reaches the volume's z band
     const bool same = __all((int)r.swap == __builtin_amdgcn_readfirstlane((int)r.swap));
-    // (the ordered walk hands pieces over when any lane crosses a slice, in range or not)
-    float slope = (ORDERED ? active && r.hit : klo <= khi) ? run_slope(r) : 0.0f;
+    int nb = 0;
+    if constexpr (RUNS) {
+        // (the ordered walk hands pieces over when any lane crosses a slice, in range or not)
+        float slope = (ORDERED ? active && r.hit : klo <= khi) ? run_slope(r) : 0.0f;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) slope = fmaxf(slope, __shfl_xor(slope, o, 64));
-    int nb = same && (size_t)g.N * g.N * g.Nz <= (size_t)RunAcc<VoxT>::kOut ? run_block_steps(g, slope) : 0;
-    nb = __builtin_amdgcn_readfirstlane(nb);
-    if (ORDERED && !g.aligned) nb = 0;
-    if (nb > 0) {
+        for (int o = 32; o >= 1; o >>= 1) slope = fmaxf(slope, __shfl_xor(slope, o, 64));
+        if (same && run_walk<VoxT>(g)) nb = __builtin_amdgcn_readfirstlane(run_block_steps(g, slope));
+        if (nb < kRunSteps<ORDERED> || (ORDERED && !g.aligned)) nb = 0;
+    }
+    if (RUNS && nb > 0) {
         if constexpr (ORDERED) {
             OrderedAcc<VoxT> acc(vox, g);
             walk_runs_ordered(g, r, active, kmin, kmax, nb, acc, &lds->ordered);
@@ -498,7 +522,7 @@ __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double s
         acc.Nz = g.Nz;
 #pragma unroll
         for (int m = 0; m < VCBCT_MAX_MAT; ++m) acc.L[m] = 0.0f;
-        traverse_lane(g, r, active, kmin, kmax, acc, ORDERED && same ? &lds->table : nullptr);
+        traverse_lane(g, r, active, kmin, kmax, acc, same ? &lds->table : nullptr);
         acc.finish();
 #pragma unroll
         for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
@@ -716,7 +740,7 @@ bool tile_shape_valid(const TileShape& s) {
 }
 
 // One wave: 64 detector rows [64 rg, 64 rg + 64) of column jj at angle a.  Wave-uniform arguments.
-template <int MODE, class VoxT>
+template <int MODE, class VoxT, bool RUNS>
 __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __restrict__ tab,
                                              const VoxT* __restrict__ vox, const double* __restrict__ mu,
                                              const double* __restrict__ pdf, const float* __restrict__ muf,
@@ -738,7 +762,7 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
         return;
     }
     float L[VCBCT_MAX_MAT];
-    const double leng = sum_wave<false>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
+    const double leng = sum_wave<false, RUNS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
     if (!active) return;
 
     if (MODE == VCBCT_MODE_LINEINT) {
@@ -803,8 +827,8 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
 }
 
 // WPB waves per block (TileShape: rgb * cols); the block's waves share nothing but the LDS allocation.
-template <int MODE, class VoxT, int WPB>
-__global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_RUN void k_forward(ProjGeom g, const double* __restrict__ tab,
+template <int MODE, class VoxT, int WPB, bool RUNS>
+__global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_FWD(MODE, RUNS) void k_forward(ProjGeom g, const double* __restrict__ tab,
                                                                  const VoxT* __restrict__ vox,
                                                                  const double* __restrict__ mu,
                                                                  const double* __restrict__ pdf,
@@ -815,7 +839,7 @@ __global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_RUN void k_forward(ProjGeom g
     __shared__ WalkLds steps[WPB];
     const Tile t = tile_map(tm, nA);
     if (t.col >= g.W || t.a >= nA || t.rg * 64 >= g.H) return;  // wave out of range: uniform exit
-    forward_wave<MODE, VoxT>(g, tab, vox, mu, pdf, muf, pdff, NE, inv_xf, nl, a0 + t.a, t.rg, t.col, out, aux,
+    forward_wave<MODE, VoxT, RUNS>(g, tab, vox, mu, pdf, muf, pdff, NE, inv_xf, nl, a0 + t.a, t.rg, t.col, out, aux,
                              &steps[threadIdx.x >> 6]);
 }
 
@@ -861,7 +885,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_RUN void k_forward_batch(const Bat
             const int a = P.split ? q * P.pang + al : al;
             const int jj = P.split ? cl : q * P.pcols + cl;
             if (jj >= P.g.W || a >= P.g.nAng) continue;
-            forward_wave<VCBCT_MODE_INTENSITY, VoxT>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
+            forward_wave<VCBCT_MODE_INTENSITY, VoxT, true>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
                                                      P.inv_xf, P.g.nmat, a, rg, jj, P.out, nullptr,
                                                      &steps[threadIdx.x >> 6]);
         }
@@ -884,7 +908,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_RUN void k_forward_flat(const Batc
     const BatchProblem& P = pr[lo];
     const Tile t = tile_map(P.tm, P.g.nAng, b - P.block_start);
     if (t.col >= P.g.W || t.a >= P.g.nAng || t.rg * 64 >= P.g.H) return;  // wave out of range: uniform exit
-    forward_wave<VCBCT_MODE_INTENSITY, VoxT>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
+    forward_wave<VCBCT_MODE_INTENSITY, VoxT, true>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
                                              P.inv_xf, P.g.nmat, t.a, t.rg, t.col, P.out, nullptr,
                                              &steps[threadIdx.x >> 6]);
 }
@@ -985,8 +1009,8 @@ struct ScatterG {
 
 // VoxT float4: the FP32 maps (mu / muf the material tables, nl = nmat); float2 / Ch4: their channel volume
 // (mu / muf the channel tables, nl = nch).
-template <int MODE, class VoxT>
-__global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(ProjGeom g, const double* __restrict__ tab,
+template <int MODE, class VoxT, bool RUNS>
+__global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE, RUNS) void k_adjoint_coef(ProjGeom g, const double* __restrict__ tab,
                                                       const VoxT* __restrict__ vox, const double* __restrict__ mu,
                                                       const double* __restrict__ pdf, const float* __restrict__ muf,
                                                       const double* __restrict__ ch, int nch, int NE, double inv_xf,
@@ -1005,7 +1029,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
     const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
                  yc = ldk(tab, 3 * g.nAng + a);
     float L[VCBCT_MAX_MAT];
-    sum_wave<MODE == VCBCT_ADJ_LOSS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
+    sum_wave<MODE == VCBCT_ADJ_LOSS, RUNS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
 
     double lossc = 0.0;
     if (active) {
@@ -1069,8 +1093,8 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE) void k_adjoint_coef(Pro
 // the sum over the spectra, c_k = sum_s 2 (p_s - t_s) chbar_sk / xf, so that one scatter serves all spectra.
 // NCH: the channel count (the arrays of the spectral loop stay in registers).  VoxT float4: the FP32 maps (the
 // exponents over the material tables); float2 / Ch4: the joint basis's channel volume (over the channel tables).
-template <int NCH, class VoxT>
-__global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(ProjGeom g, const double* __restrict__ tab,
+template <int NCH, class VoxT, bool RUNS>
+__global__ __launch_bounds__(256) VCBCT_WAVES_MULTI(RUNS) void k_adjoint_coef_multi(ProjGeom g, const double* __restrict__ tab,
                                                                          const VoxT* __restrict__ vox, SpecSet ss,
                                                                          double inv_xf, TileMap tm,
                                                                          const float* __restrict__ tg,
@@ -1088,7 +1112,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_ORDERED void k_adjoint_coef_multi(
     const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
                  yc = ldk(tab, 3 * g.nAng + a);
     float L[VCBCT_MAX_MAT];
-    sum_wave<true>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
+    sum_wave<true, RUNS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
 
     double lossc = 0.0;
     if (active) {
@@ -1322,15 +1346,23 @@ template <int M, class T>
 static void launch_fwd_t(int wpb, dim3 grid, hipStream_t st, const ProjGeom& g, const double* tables, const void* vox,
                          const Spectrum& sp, double inv_xf, int a0, int nA, const TileMap& tm, float* out,
                          float* aux) {
-#define VCBCT_LAUNCH_FWD(W)                                                                                  \
-    hipLaunchKernelGGL((k_forward<M, T, W>), grid, dim3(64 * W), 0, st, g, tables, (const T*)vox, sp.mu, sp.pdf, \
+#define VCBCT_LAUNCH_FWD(W, RUNS)                                                                             \
+    hipLaunchKernelGGL((k_forward<M, T, W, RUNS>), grid, dim3(64 * W), 0, st, g, tables, (const T*)vox, sp.mu, sp.pdf, \
                        sp.muf, sp.pdff, sp.NE, inv_xf, sp.nl, a0, nA, tm, out, aux)
     if constexpr (M == VCBCT_MODE_INTENSITY || M == VCBCT_MODE_LOGPROJ) {
-        if (wpb == 2) VCBCT_LAUNCH_FWD(2);
-        else if (wpb == 8) VCBCT_LAUNCH_FWD(8);
-        else VCBCT_LAUNCH_FWD(4);
+        if (run_walk<T>(g)) {
+            if (wpb == 2) VCBCT_LAUNCH_FWD(2, true);
+            else if (wpb == 8) VCBCT_LAUNCH_FWD(8, true);
+            else VCBCT_LAUNCH_FWD(4, true);
+        } else {
+            if (wpb == 2) VCBCT_LAUNCH_FWD(2, false);
+            else if (wpb == 8) VCBCT_LAUNCH_FWD(8, false);
+            else VCBCT_LAUNCH_FWD(4, false);
+        }
+    } else if constexpr (M == VCBCT_MODE_LINEINT) {
+        VCBCT_LAUNCH_FWD(4, true);
     } else {
-        VCBCT_LAUNCH_FWD(4);
+        VCBCT_LAUNCH_FWD(4, false);
     }
 #undef VCBCT_LAUNCH_FWD
 }
@@ -1558,9 +1590,15 @@ static int launch_coef(const ProjGeom& g, const double* tables, const void* vox,
     TileMap tm;
     const long nb = tile_map_host(g, g.nAng, s, tm);
     if (nb < 0) return fail(VCBCT_EINVAL, "adjoint: launch too large");
-#define VCBCT_LAUNCH_COEF(M, T)                                                                               \
-    hipLaunchKernelGGL((k_adjoint_coef<M, T>), dim3((unsigned)nb), dim3(256), 0, st, g, tables, (const T*)vox,  \
+#define VCBCT_LAUNCH_COEF_R(M, T, R)                                                                             \
+    hipLaunchKernelGGL((k_adjoint_coef<M, T, R>), dim3((unsigned)nb), dim3(256), 0, st, g, tables, (const T*)vox, \
                        sp.mu, sp.pdf, sp.muf, sp.ch, sp.nch, sp.NE, inv_xf, sp.nl, tm, tg, coef, loss)
+    // (the ordered walk serves aligned plane grids)
+#define VCBCT_LAUNCH_COEF(M, T)                                                                         \
+    do {                                                                                                 \
+        if (run_walk<T>(g) && ((M) != VCBCT_ADJ_LOSS || g.aligned)) VCBCT_LAUNCH_COEF_R(M, T, true);      \
+        else VCBCT_LAUNCH_COEF_R(M, T, false);                                                           \
+    } while (0)
     if (mode == VCBCT_ADJ_LOSS) {
         if (vox_kind == VOX_CH2) VCBCT_LAUNCH_COEF(VCBCT_ADJ_LOSS, float2);
         else if (vox_kind == VOX_CH4) VCBCT_LAUNCH_COEF(VCBCT_ADJ_LOSS, Ch4);
@@ -1571,6 +1609,7 @@ static int launch_coef(const ProjGeom& g, const double* tables, const void* vox,
         else VCBCT_LAUNCH_COEF(VCBCT_ADJ_UPSTREAM, float4);
     }
 #undef VCBCT_LAUNCH_COEF
+#undef VCBCT_LAUNCH_COEF_R
     VCBCT_HIP(hipGetLastError());
     return 0;
 }
@@ -1581,9 +1620,14 @@ static int launch_coef_multi(const ProjGeom& g, const double* tables, const void
     TileMap tm;
     const long nb = tile_map_host(g, g.nAng, s, tm);
     if (nb < 0) return fail(VCBCT_EINVAL, "adjoint: launch too large");
-#define VCBCT_LAUNCH_MULTI(C, T)                                                                                \
-    hipLaunchKernelGGL((k_adjoint_coef_multi<C, T>), dim3((unsigned)nb), dim3(256), 0, st, g, tables,          \
+#define VCBCT_LAUNCH_MULTI_R(C, T, R)                                                                           \
+    hipLaunchKernelGGL((k_adjoint_coef_multi<C, T, R>), dim3((unsigned)nb), dim3(256), 0, st, g, tables,         \
                        (const T*)vox, ss, inv_xf, tm, targets, coef, loss)
+#define VCBCT_LAUNCH_MULTI(C, T)                                           \
+    do {                                                                   \
+        if (run_walk<T>(g) && g.aligned) VCBCT_LAUNCH_MULTI_R(C, T, true); \
+        else VCBCT_LAUNCH_MULTI_R(C, T, false);                            \
+    } while (0)
     if (vox_kind == VOX_CH2) {
         if (ss.nch == 1) VCBCT_LAUNCH_MULTI(1, float2);
         else if (ss.nch == 2) VCBCT_LAUNCH_MULTI(2, float2);
@@ -1604,6 +1648,7 @@ static int launch_coef_multi(const ProjGeom& g, const double* tables, const void
         }
     }
 #undef VCBCT_LAUNCH_MULTI
+#undef VCBCT_LAUNCH_MULTI_R
     VCBCT_HIP(hipGetLastError());
     return 0;
 }

@@ -177,18 +177,17 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
     // the position of plane f = mm, z = (nzm - mm) t, in the step walk's expression (a plane met on the way to z = 0
     // is formed from the one after it, as the reference forms it)
     auto plane_at = [&](int mm) -> double {
-        const int pz = nzm - mm;
-        const double zb = pz * sgn > 0 ? (double)(pz - sgn) * g.t + (double)sgn * g.t : (double)pz * g.t;
+        const int pz = nzm - mm, from = pz * sgn > 0 ? sgn : 0;
+        const double zb = (double)(pz - from) * g.t + (double)from * g.t;
         return on && fA != 0.0 ? (zb - r.sz) * duzD : 1.0e300;
     };
     int il = (int)fmin(fmax(floor((D0 + 1e-3 * g.s) * fA + (r.sz * c.ninv_t + c.nzm)), -1.0e9), 1.0e9);
     double dnext = plane_at(il + up);
-    if (on && fA != 0.0) {  // (a plane within the first thousandth of the first step is met in that step)
+    {  // (a plane within the first thousandth of the first step is met in that step)
         const double Dprev = plane_at(il + up - sgn);
-        if (Dprev > D0) {
-            il -= sgn;
-            dnext = Dprev;
-        }
+        const bool back = on && fA != 0.0 && Dprev > D0;
+        il -= back ? sgn : 0;
+        dnext = back ? Dprev : dnext;
     }
     auto slice_off = [&](int i) -> int {  // cell offset of logical slice i, or out of the volume
         return on && (unsigned)(i + 1) <= (unsigned)g.Nz ? (i < 0 ? 0 : i) : (int)Acc::kOut;
@@ -397,19 +396,18 @@ __host__ __device__ __forceinline__ void walk_runs_ordered(const ProjGeom& g, co
     const int up = fA > 0.0 ? 1 : 0, sgn = fA > 0.0 ? 1 : -1;
     const int nzm = (int)c.nzm;
     auto plane_at = [&](int mm) -> double {  // as in walk_runs
-        const int pz = nzm - mm;
-        const double zb = pz * sgn > 0 ? (double)(pz - sgn) * g.t + (double)sgn * g.t : (double)pz * g.t;
+        const int pz = nzm - mm, from = pz * sgn > 0 ? sgn : 0;
+        const double zb = (double)(pz - from) * g.t + (double)from * g.t;
         return on && fA != 0.0 ? (zb - r.sz) * duzD : 1.0e300;
     };
     const double D0 = b0 * r.pha;
     int il = (int)fmin(fmax(floor((D0 + 1e-3 * g.s) * fA + (r.sz * c.ninv_t + c.nzm)), -1.0e9), 1.0e9);
     double dnext = plane_at(il + up);
-    if (on && fA != 0.0) {
+    {
         const double Dprev = plane_at(il + up - sgn);
-        if (Dprev > D0) {
-            il -= sgn;
-            dnext = Dprev;
-        }
+        const bool back = on && fA != 0.0 && Dprev > D0;
+        il -= back ? sgn : 0;
+        dnext = back ? Dprev : dnext;
     }
     auto slice_off = [&](int i) -> int {
         return on && (unsigned)(i + 1) <= (unsigned)g.Nz ? (i < 0 ? 0 : i) : (int)Acc::kOut;
