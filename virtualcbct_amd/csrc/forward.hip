@@ -379,7 +379,7 @@ template <class VoxT>
 struct RunAcc {
     typedef RunRec<VoxT> Q;
     static constexpr int kOut = (int)(0x80000000u >> Q::kShift);
-        // gathers in flight per wave (512x512x128 / 360 angles: 10.6 ms with 8, 10.6 with 4; 320x320x77 / 120 angles: 2.12
+    // gathers in flight per wave (512x512x128 / 360 angles: 10.6 ms with 8, 10.6 with 4; 320x320x77 / 120 angles: 2.12
     // against 2.25 ms); the two-load FP32 record half of that
     static constexpr int kBatch = sizeof(Q) <= 16 ? 8 : 4;
     __amdgpu_buffer_rsrc_t buf;
@@ -396,31 +396,29 @@ struct RunAcc {
 #pragma unroll
         for (int m = 0; m < Q::kTerms; ++m) L[m] += q.term(m) * len;
     }
-    // pieces [pa, pb) of the list: before first_new to offset zo, the rest to zn; the lane's length of piece px is lo
-    __device__ __forceinline__ void run(const PieceRec* p, int pa, int pb, int px, int first_new, float lo, int zo,
-                                        int zn, float K) {
+    // Pieces [i, i + B) of the list, those past pb off the volume (runs.h's run_gaps).
+    template <int B>
+    __device__ __forceinline__ void batch(const PieceRec* p, int i, int pb, int first_new, int gap_end, int zo, int zn,
+                                          float K) {
+        PieceRec t[B];
+        Q q[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) t[b] = p[i + b < pb ? i + b : pb - 1];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int z = i + b < first_new ? zo : i + b >= gap_end ? zn : kOut;
+            load(t[b].cb + (i + b < pb ? z : kOut), q[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+            add(q[b], i + b < pb ? t[b].len * K : 0.0f);
+    }
+    __device__ __forceinline__ void run_gaps(const PieceRec* p, int pa, int pb, int first_new, int gap_end, int zo,
+                                             int zn, double K) {
+        const float Kf = (float)K;
         int i = pa;
-        for (; i + kBatch <= pb; i += kBatch) {
-            PieceRec t[kBatch];
-            Q q[kBatch];
-#pragma unroll
-            for (int b = 0; b < kBatch; ++b) t[b] = p[i + b];
-#pragma unroll
-            for (int b = 0; b < kBatch; ++b) load(t[b].cb + (i + b < first_new ? zo : zn), q[b]);
-#pragma unroll
-            for (int b = 0; b < kBatch; ++b) add(q[b], i + b == px ? lo : t[b].len * K);
-        }
-        if (i < pb) {  // the rest as one batch: past the end, the last piece again with length 0
-            PieceRec t[kBatch - 1];
-            Q q[kBatch - 1];
-#pragma unroll
-            for (int b = 0; b < kBatch - 1; ++b) t[b] = p[i + b < pb ? i + b : pb - 1];
-#pragma unroll
-            for (int b = 0; b < kBatch - 1; ++b)
-                load(t[b].cb + ((i + b < pb ? i + b : pb - 1) < first_new ? zo : zn), q[b]);
-#pragma unroll
-            for (int b = 0; b < kBatch - 1; ++b) add(q[b], i + b >= pb ? 0.0f : i + b == px ? lo : t[b].len * K);
-        }
+        for (; i + kBatch <= pb; i += kBatch) batch<kBatch>(p, i, i + kBatch, first_new, gap_end, zo, zn, Kf);
+        if (i < pb) batch<kBatch - 1>(p, i, pb, first_new, gap_end, zo, zn, Kf);
     }
 };
 
@@ -437,13 +435,13 @@ struct OrderedAcc : RunAcc<VoxT> {
         for (int i = pa; i < pb; i += kBatch) {
             OrderedPiece t[kBatch];
             Q q[kBatch];
-            // (past the end: the last piece again, with length 0 off the volume)
+            // (past the end: the last piece's column with length 0, off the volume)
 #pragma unroll
             for (int b = 0; b < kBatch; ++b) t[b] = p[i + b < pb ? i + b : pb - 1];
 #pragma unroll
             for (int b = 0; b < kBatch; ++b) {
-                const int k = i + b < pb ? i + b : pb - 1;
-                this->load(t[b].cb + (k < first_new || k == px ? zo : zn), q[b]);
+                const int z = i + b < first_new || i + b == px ? zo : zn;
+                this->load(t[b].cb + (i + b < pb ? z : RunAcc<VoxT>::kOut), q[b]);
             }
 #pragma unroll
             for (int b = 0; b < kBatch; ++b)

@@ -5,13 +5,14 @@
 // only, and a lane changes slice rarely (the cone's slopes: every 20 to 60 steps on a 0.5 mm / 1 mm grid).  So the
 // walk keeps, per lane, the slice it is in and the position of its next slice plane, and takes the xy pieces
 // of up to `nb` steps at a time, few enough that no lane meets two slice planes in them:
-//  - the lanes that meet a plane in the block find the piece that holds it, and its two parts;
-//  - main loop: every piece up to that one goes to the lane's slice, the rest to the next one, with the piece's length
-//    except for the one that holds the plane (its first part).  Column and length come from the wave's LDS table (one
-//    8-byte broadcast read), so a piece takes seven vector instructions (two compares and selects against the
-//    uniform piece number, one address, two multiply-adds for two channels), against ~90 when each step formed
-//    its own slice indices and crossings;
-//  - the second parts are charged, all lanes of the block together.
+//  - the lanes that meet a plane in the block find the piece that holds it, and gather its two parts for themselves;
+//  - main loop: every piece before that one goes to the lane's slice, those after it to the next one.  Column and
+//    length come from the wave's LDS table (one 8-byte broadcast read), so a piece takes nine vector instructions (two
+//    compares and selects against the uniform piece number, one address, two for the length, two multiply-adds for
+//    two channels), against ~90 when each step formed its own slice indices and crossings;
+//  - the parts are charged, all lanes of the block together.
+// Nothing is read of a voxel that the lane does not charge: the piece that holds the plane, and the places past the end of a
+// batch of gathers, are read off the volume (zeros), as a length of 0 would make a NaN of an infinite voxel.
 // The reference's rules hold as in the step walk: midpoint truncation (slice 0 takes the truncated (-1, 0) range
 // too), the z = 0 plane splits nothing (the whole piece goes to its midpoint's slice), the inscribed-circle test at
 // the midpoint, and equal crossing distances charge the whole chord once.  Where those need a part's own midpoint
@@ -132,9 +133,24 @@ __host__ __device__ __forceinline__ int run_block_steps(const ProjGeom& g, float
     return n >= 64.0 ? 64 : (n >= 1.0 ? (int)n : 0);
 }
 
+// Pieces [pa, pb) of the list: before first_new from slice offset zo, from gap_end on from zn, none between.  By the
+// accumulator's own form, or in two passes.
+template <class Acc>
+__host__ __device__ __forceinline__ auto run_gaps(Acc& acc, const PieceRec* p, int pa, int pb, int first_new,
+                                                  int gap_end, int zo, int zn, double K, int)
+    -> decltype(acc.run_gaps(p, pa, pb, first_new, gap_end, zo, zn, K)) {
+    acc.run_gaps(p, pa, pb, first_new, gap_end, zo, zn, K);
+}
+template <class Acc>
+__host__ __device__ __forceinline__ void run_gaps(Acc& acc, const PieceRec* p, int pa, int pb, int first_new,
+                                                  int gap_end, int zo, int zn, double K, long) {
+    acc.run(p, pa, pb, INT_MAX, first_new, 0.0f, zo, (int)Acc::kOut, K);
+    acc.run(p, pa, pb, INT_MAX, gap_end, 0.0f, (int)Acc::kOut, zn, K);
+}
+
 // Walks plane steps [kmin, kmax] of one wave (lanes with a common xy path, `nb` from run_block_steps).
-// Acc: float accumulator with load(cell, q) (cell outside the volume: zeros), add(q, length), run() for a list of
-// pieces, a record type Q, and kOut, a cell offset that no column brings back into the volume.
+// Acc: float accumulator with load(cell, q) (cell outside the volume: zeros), add(q, length), run_gaps() or run() for a
+// list of pieces, a record type Q, and kOut, a cell offset that no column brings back into the volume.
 template <bool ALIGNED, class Acc>
 __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayCtx& r_in, bool active, int kmin,
                                                    int kmax, int nb, Acc& acc, RunLds* lds) {
@@ -154,7 +170,6 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
 #endif
     constexpr bool kEarly = sizeof(typename Acc::Q) <= 8;
     const bool on = active && r.hit;
-    const float K = (float)r.K;
     const ChargeC c = charge_consts(g, r);
     const double u0 = r.uin;
     const double v0 = (u0 - r.su) * r.dv + r.sv;
@@ -200,7 +215,7 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
         {
             RunStep t;
             PieceRec p0, p1;
-                        bool has0, has1;
+            bool has0, has1;
             bool ok = make_run_step<ALIGNED>(g, r, c, k + lane, t, p0, p1, has0, has1) && k + lane <= kmax;
             const unsigned long long bad = __ballot(!ok);
             nsteps = bad ? __ffsll((long long)bad) - 1 : 64;
@@ -224,7 +239,7 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
             for (int l = 0; l < 64; ++l) {
                 RunStep t;
                 PieceRec p0, p1;
-                                bool has0, has1;
+                bool has0, has1;
                 const bool ok = make_run_step<ALIGNED>(g, r, c, k + l, t, p0, p1, has0, has1) && k + l <= kmax;
                 if (!ok && nsteps == 64) nsteps = l;
                 t.flags |= total << RUN_SHIFT;
@@ -247,12 +262,11 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
 #endif
             const bool cross = dnext < r.pha * lds->dk[ke - 1];
             const int zo = slice_off(il), zn = slice_off(il + sgn);
-            // Crossing lanes: the step and the piece that hold the plane, the piece's two parts; px its number in
-            // the list (pieces from px + 1, or from px where it is not listed, go to the next slice).
-            int px = INT_MAX, first_new = INT_MAX;
-            float lo = 0.0f, ln = 0.0f;
+            // Crossing lanes: the step and the piece that hold the plane.  The piece is left out of the list's sums, pieces
+            // from gap_end on go to the next slice, and the two parts beside the plane are gathered for themselves.
+            int first_new = INT_MAX, gap_end = INT_MAX;
             bool special = false, tie = false;
-            typename Acc::Q v1, v2;  // the parts beside the list
+            typename Acc::Q v1, v2;  // the parts
             int c1 = (int)Acc::kOut, c2 = c1;
             float l1 = 0.0f, l2 = 0.0f;
             if (any_lane(cross)) {
@@ -271,10 +285,13 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
                     const bool zero = il + up == nzm;  // the z = 0 plane splits nothing: whole, by the midpoint
                     special = !zero && ((t.flags & RUN_SPECIAL) || tie);
                     const double at = zero ? ((a + b) * 0.5 < dnext ? b : a) : dnext;
-                    if (listed) {
-                        px = first_new++;
-                        lo = special ? 0.0f : (float)(fmax(at - a, 0.0) * r.K);
-                        ln = special ? 0.0f : (float)(fmax(b - at, 0.0) * r.K);
+                    gap_end = first_new + (listed ? 1 : 0);
+                    if (listed && !special) {  // (a part of no length is not charged: its voxel may be infinite)
+                        const int cb = lds->pieces[first_new].cb;
+                        l1 = (float)(fmax(at - a, 0.0) * r.K);
+                        l2 = (float)(fmax(b - at, 0.0) * r.K);
+                        c1 = l1 > 0.0f ? cb + zo : (int)Acc::kOut;
+                        c2 = l2 > 0.0f ? cb + zn : (int)Acc::kOut;
                     }
                 }
                 // The parts' gathers go out before the block's and are added after it (kEarly, two-channel records): waiting
@@ -290,33 +307,24 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
                     const double uz = r.pha * dnext + r.su, uv = t.dv + r.su;
                     const double uk = plane_u(r, k + kc, g.s), ub0 = plane_u(r, k + kc - 1, g.s);
                     const Seg s1 = make_seg<false, false>(g, r, c, tie || z0 ? ub0 : uv, tie ? uk : uz, on && special, 0, false);
-                    c1 = s1.ok ? s1.cell : (int)Acc::kOut;
-                    l1 = s1.ok ? (float)s1.rr : 0.0f;
                     const Seg s2 = make_seg<false, false>(g, r, c, uz, z0 && splitv ? uv : uk, on && special && !tie, 0, false);
-                    c2 = s2.ok ? s2.cell : (int)Acc::kOut;
-                    l2 = s2.ok ? (float)s2.rr : 0.0f;
-                    if (any_lane(special && tie)) {  // the pieces of such lanes that the main loop will charge
-#pragma unroll 1
-                        for (int q = 0; q < 2; ++q) {
-                            const int p0 = t.flags >> RUN_SHIFT, p = p0 + (q && (t.flags & STEP_OK0) ? 1 : 0);
-                            const bool take = special && tie && (t.flags & (q ? STEP_OK1 : STEP_OK0)) && p != px;
-                            const PieceRec pr = lds->pieces[take ? p : 0];
-                            typename Acc::Q v;
-                            acc.load(take ? pr.cb + (p < first_new ? zo : zn) : (int)Acc::kOut, v);
-                            acc.add(v, take ? -(pr.len * K) : 0.0f);
+                    if (special) {
+                        c1 = s1.ok ? s1.cell : (int)Acc::kOut;
+                        l1 = s1.ok ? (float)s1.rr : 0.0f;
+                        c2 = s2.ok ? s2.cell : (int)Acc::kOut;
+                        l2 = s2.ok ? (float)s2.rr : 0.0f;
+                        if (tie) {  // both pieces are left out
+                            first_new = t.flags >> RUN_SHIFT;
+                            gap_end = first_new + (t.flags & STEP_OK0 ? 1 : 0) + (t.flags & STEP_OK1 ? 1 : 0);
                         }
                     }
-                }
-                if (ln > 0.0f) {  // (not in lanes with special parts)
-                    c2 = lds->pieces[px].cb + zn;
-                    l2 = ln;
                 }
                 if (kEarly) {
                     acc.load(c1, v1);
                     acc.load(c2, v2);
                 }
             }
-            acc.run(lds->pieces, pa, pb, px, first_new, lo, zo, zn, K);
+            run_gaps(acc, lds->pieces, pa, pb, first_new, gap_end, zo, zn, r.K, 0);
             if (any_lane(cross)) {
                 if (!kEarly) {
                     acc.load(c1, v1);
