@@ -399,7 +399,7 @@ struct RunAcc {
     // Pieces [i, i + B) of the list, those past pb off the volume (runs.h's run_gaps).
     template <int B>
     __device__ __forceinline__ void batch(const PieceRec* p, int i, int pb, int first_new, int gap_end, int zo, int zn,
-                                          float K) {
+                                          double K) {
         PieceRec t[B];
         Q q[B];
 #pragma unroll
@@ -411,14 +411,13 @@ struct RunAcc {
         }
 #pragma unroll
         for (int b = 0; b < B; ++b)
-            add(q[b], i + b < pb ? t[b].len * K : 0.0f);
+            add(q[b], i + b < pb ? (float)(t[b].len * K) : 0.0f);
     }
     __device__ __forceinline__ void run_gaps(const PieceRec* p, int pa, int pb, int first_new, int gap_end, int zo,
                                              int zn, double K) {
-        const float Kf = (float)K;
         int i = pa;
-        for (; i + kBatch <= pb; i += kBatch) batch<kBatch>(p, i, i + kBatch, first_new, gap_end, zo, zn, Kf);
-        if (i < pb) batch<kBatch - 1>(p, i, pb, first_new, gap_end, zo, zn, Kf);
+        for (; i + kBatch <= pb; i += kBatch) batch<kBatch>(p, i, i + kBatch, first_new, gap_end, zo, zn, K);
+        if (i < pb) batch<kBatch - 1>(p, i, pb, first_new, gap_end, zo, zn, K);
     }
 };
 

@@ -7,7 +7,7 @@
 // of up to `nb` steps at a time, few enough that no lane meets two slice planes in them:
 //  - the lanes that meet a plane in the block find the piece that holds it, and gather its two parts for themselves;
 //  - main loop: every piece before that one goes to the lane's slice, those after it to the next one.  Column and
-//    length come from the wave's LDS table (one 8-byte broadcast read), so a piece takes nine vector instructions (two
+//    length come from the wave's LDS table (one 16-byte broadcast read), so a piece takes nine vector instructions (two
 //    compares and selects against the uniform piece number, one address, two for the length, two multiply-adds for
 //    two channels), against ~90 when each step formed its own slice indices and crossings;
 //  - the parts are charged, all lanes of the block together.
@@ -20,8 +20,9 @@
 // step walk forms its segments.
 // What bounds it: on the 512x512x128 / 360-angle projection the gathers' traffic beyond L2 (7.7e10 bytes at 7.4 TB/s);
 // the step walk took 20.7 ms there, bound by vector issue (1.19e10 wave-instructions, now 4.5e9), this walk 10.5 ms.
-// A piece's length is its extent along the major axis times the ray's length factor, multiplied per piece as the step
-// walk does: FP32 sums of equal terms (a constant map) round one way, and by the terms' own digits, so lengths scaled
+// A piece's length is its extent along the major axis times the ray's length factor, formed in FP64 and rounded once per
+// piece as the step walk does (extent and factor rounded to FP32 first shift a whole ray by up to 6e-8; the full scan takes
+// the same 10.7 ms, 320x320x77 at 0.977 mm / 120 angles 1.87 against 1.80 ms, six u16 maps 1.47 against 1.50): FP32 sums of equal terms (a constant map) round one way, and by the terms' own digits, so lengths scaled
 // once at the end would leave a log projection 1e-7 off the step walk's there.
 #pragma once
 
@@ -29,10 +30,10 @@
 
 namespace vcbct {
 
-// One xy piece: its voxel column and its extent along the major axis.
+// One xy piece: its extent along the major axis and its voxel column.
 struct PieceRec {
-    int cb;
-    float len;
+    double len;
+    int cb, pad;
 };
 
 // One step: the positions of its end plane and minor crossing relative to the source (as StepRec), and in flags
@@ -50,11 +51,7 @@ struct RunLds {
     PieceRec pieces[128];
 };
 
-// A piece of the ordered walk: its length per unit of the major axis in FP64, its voxel column.
-struct OrderedPiece {
-    double len;
-    int cb, pad;
-};
+typedef PieceRec OrderedPiece;  // (the ordered walk's)
 struct OrderedLds {
     WaveLds table;
     OrderedPiece pieces[128];
@@ -116,8 +113,8 @@ __host__ __device__ __forceinline__ bool make_run_step(const ProjGeom& g, const 
     t.dv = dv;
     p0.cb = (int)((unsigned)imin0 * (unsigned)c.mstride + (unsigned)imaj0 * (unsigned)c.majmul);
     p1.cb = (int)((unsigned)imin1 * (unsigned)c.mstride + (unsigned)imaj1 * (unsigned)c.majmul);
-    p0.len = (float)fabs(d1 - dup);
-    p1.len = (float)fabs(duk - dv);
+    p0.len = fabs(d1 - dup);
+    p1.len = fabs(duk - dv);
     t.flags = (splitv ? STEP_SPLITV : 0) | (has0 ? STEP_OK0 : 0) | (has1 ? STEP_OK1 : 0) |
               (circ || !ALIGNED ? RUN_SPECIAL : 0);
     return inprev;
