@@ -660,8 +660,8 @@ __device__ __forceinline__ double mubar_opaque(const float (&L)[VCBCT_MAX_MAT], 
     return xmin - log(se / sw);
 }
 
-// 2^x as the hardware gives it: exp2f without its steps for results below 2^-126, which come out as zero here.  (Such
-// terms are 1e-8 of the smallest sum that is not re-formed in FP64.)
+// 2^x as the hardware gives it: exp2f without its steps for results below 2^-126, which come out as zero here.  (The
+// spectral sums are re-formed in FP64 where they are below 1e-30 of the spectrum's, 1e8 times such terms.)
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
 __device__ __forceinline__ bool all_zero(const float (&L)[VCBCT_MAX_MAT]) {
@@ -786,20 +786,17 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
             for (int e = 0; e < NE; ++e) s += (float)(ldk(pdf, e) * 1.0 * leng);
         } else {
             const float k2 = (float)(-inv_xf * 1.4426950408889634);
-            float Lk[VCBCT_MAX_MAT];
-#pragma unroll
-            for (int m = 0; m < VCBCT_MAX_MAT; ++m) Lk[m] = L[m] * k2;
 #pragma unroll 4
             for (int e = 0; e < NE; ++e) {
                 float tr = 0.0f;
 #pragma unroll
                 for (int m = 0; m < NT; ++m)
-                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), Lk[m], tr);
-                s = fmaf(ldk(pdff, e), exp2_fast(tr), s);
+                    if (m < nl) tr = fmaf(ldk(muf, m * NE + e), L[m], tr);
+                s = fmaf(ldk(pdff, e), exp2_fast(tr * k2), s);
             }
             s *= (float)leng;
-            // opaque ray: the FP32 exponentials underflow; the reference's own FP64 terms instead
-            if (s < 1e-30f) s = intensity_exact(L, nl, mu, pdf, NE, inv_xf, leng);
+            // opaque ray (the FP32 exponentials underflow, or the sum does): the reference's own FP64 terms instead
+            if (s < 1e-30f * fmaxf(1.0f, (float)(leng * ldk(pdf, NE)))) s = intensity_exact(L, nl, mu, pdf, NE, inv_xf, leng);
         }
         stg(out, o, s);
     } else {  // VCBCT_MODE_LOGPROJ: p = -log(sum_e pdf_e e^{-mu.L/xf} / sum_e pdf_e); FP32 terms, FP64 sums
