@@ -109,8 +109,9 @@ int vcbct_projector_set_tile(vcbct_projector* p, int row_groups, int cols, int o
 /* The same for the traversal kernels of the adjoint (vcbct_projector_adjoint, _adjoint_upstream,
  * _logproj_backward_saved, _multi_loss_grad: the coefficient kernel and the scatter), whose workgroups are
  * 4 waves (row_groups * cols = 4).  row_groups = 0 (the default): autotuned per geometry, and the scatter by
- * voxel tiles where the geometry has at least 4e7 ray steps; below that ray by ray, tuned on the caller's own
- * coefficients with the gradient cleared again after the timing launches.  A fixed shape selects the ray-ordered
+ * voxel tiles where the geometry has at least 4e7 ray steps (with three channels or more also two angles to a
+ * workgroup, and slices not too thin for it); else ray by ray, tuned on the caller's own coefficients with the
+ * gradient cleared again after the timing launches.  A fixed shape selects the ray-ordered
  * scatter.  The scatter's floating-point additions are unordered under every shape. */
 int vcbct_projector_set_adjoint_tile(vcbct_projector* p, int row_groups, int cols, int order, int split);
 /* The shape the last intensity / log-projection launch used: shape4 = {row_groups, cols, order, split}

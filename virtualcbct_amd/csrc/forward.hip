@@ -1717,14 +1717,14 @@ static int scatter_shape(const ProjGeom& g, const double* tables, const float* c
 }
 
 size_t adjoint_coef_bytes(const ProjGeom& g) {
-    return align16((size_t)g.nAng * g.H * g.W * g.nmat * sizeof(float)) + (scatter_by_tiles(g) ? scatter_work_bytes(g) : 0);
+    return align16((size_t)g.nAng * g.H * g.W * g.nmat * sizeof(float)) + (scatter_by_tiles(g, 1) ? scatter_work_bytes(g) : 0);
 }
 
 // The gradient's channel planes from the coefficients: by voxel tiles (scatter.hip) and the columns that form leaves
 // over, or ray by ray where the caller fixed that form's shape or the geometry is outside the tile form's range.
 static int run_scatter(const ProjGeom& g, const double* tables, float* coef, int nch, float* grad_vox, hipStream_t st,
                        const TileShape& forced) {
-    if (forced.rgb > 0 || !scatter_by_tiles(g)) {
+    if (forced.rgb > 0 || !scatter_by_tiles(g, nch)) {
         TileShape s;
         int rc = scatter_shape(g, tables, coef, nch, grad_vox, st, forced, s);
         return rc ? rc : launch_scatter(g, tables, coef, nch, grad_vox, st, s);

@@ -528,10 +528,7 @@ __host__ __device__ __forceinline__ void walk_runs_ordered(const ProjGeom& g, co
                     }
                     // (lanes with equal crossing distances: the block ends before their step, which runs as a step)
                     if (any_lane(tie)) {
-                        int cut = tie ? kc : INT_MAX;
-#ifdef __HIP_DEVICE_COMPILE__
-                        cut = __builtin_amdgcn_readfirstlane(wave_min(cut));
-#endif
+                        const int cut = lanes_min(tie ? kc : INT_MAX);
                         slow = cut == i;
                         ie = cut;
                         if (kc >= ie) {
@@ -553,9 +550,8 @@ __host__ __device__ __forceinline__ void walk_runs_ordered(const ProjGeom& g, co
                     // crossings among them, are handed over before that step.  (Once in a block at most: after it no
                     // lane that holds a piece crosses again in the block.)
                     if (any_lane(event && held)) {
-                        int kf = event && held ? kc : INT_MAX;
+                        const int kf = lanes_min(event && held ? kc : INT_MAX);
 #ifdef __HIP_DEVICE_COMPILE__
-                        kf = __builtin_amdgcn_readfirstlane(wave_min(kf));
                         const int pf = __builtin_amdgcn_readfirstlane(tab[kf].flags) >> RUN_SHIFT;
 #else
                         const int pf = tab[kf].flags >> RUN_SHIFT;

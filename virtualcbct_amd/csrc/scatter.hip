@@ -20,8 +20,7 @@
 
 namespace vcbct {
 
-constexpr int ST = 16;  // tile side in voxels
-constexpr int SZ = 32;  // slices of a tile: 64 KB of FP64 sums a channel; a CU's 160 KB hold two, and 16 waves' lists
+constexpr int ST = kScatterSide, SZ = kScatterSlices;  // 64 KB of FP64 sums a channel; a CU's 160 KB hold two, and 16 waves' lists
 constexpr int SK = 20;  // steps of a ray in a tile: at most ST + 1 voxels along the major axis, and one each side
 
 // The xy path of the rays of one detector column at one angle (the same for all its rows), made by k_scatter_rays.
@@ -37,19 +36,6 @@ enum { SR_LIVE = 1, SR_XMAJ = 2, SR_VMOVE = 4, SR_PHA = 8, SR_DIRV = 16 };
 static size_t scatter_ray_bytes(const ProjGeom& g) { return (size_t)g.nAng * g.W * sizeof(ScatterRay); }
 size_t scatter_work_bytes(const ProjGeom& g) {
     return scatter_ray_bytes(g) + 16 + (size_t)g.nAng * g.W * sizeof(int);
-}
-
-// The tile form's range: 15-bit voxel indices, rows and columns (the latter formed in FP32 with margins of a fiftieth), a
-// slice chunk per grid layer, and a source well outside the volume (the tile's footprint on the panel is its corners'
-// projection); and at least 4e7 ray steps, as a tile costs its clearing and its final atomics whatever
-// it gathers.  Backward from saved line integrals, ray-ordered against tiles: 64x64x20 / 24 angles of 60x60 (5.5e6) 163
-// against 207 us over five channels, with 90 angles (2.1e7) 380 against 488, with 360 (8.3e7) 1272 against 1119;
-// 128x128x32 / 24 angles of 128x128 (5.0e7) 408 against 475, over two channels 256 against 217, over one 195 against 108;
-// 256x256x64 / 8 angles of 256x256 (1.3e8) 798 against 716 over five, 290 against 184 over one.
-bool scatter_by_tiles(const ProjGeom& g) {
-    const double reach = (0.5 * g.N + 1.0) * g.s * 3.0 + std::fabs(g.x_reg) + std::fabs(g.y_reg);
-    return g.N < 32768 && g.H < 32768 && g.W < 32768 && (g.Nz + SZ - 1) / SZ <= 65535 && reach < g.sad && (size_t)g.nAng * g.W < (size_t)INT_MAX &&
-           (double)g.nAng * g.H * g.W * g.N >= 4.0e7;
 }
 
 // One thread per (angle, column).
@@ -446,11 +432,8 @@ int launch_scatter_rays(const ProjGeom& g, const double* tables, void* work, hip
 int launch_scatter_tiles(const ProjGeom& g, const double* tables, const void* work, const float* coef, int nch,
                          float* gvox, hipStream_t st) {
     const int nt = (g.N + ST - 1) / ST, nzc = (g.Nz + SZ - 1) / SZ;
-    // Angle groups: at least eight blocks a CU where the angles allow it, so that the last ones leave little of the chip
-    // idle; columns split further where a block's waves would get fewer than four tasks each.
-    const long tiles = std::max(1L, (long)(0.785 * nt * nt)) * nzc;
-    const int ngroup = (int)std::min<long>(g.nAng, std::max(1L, (2048 + tiles - 1) / tiles));
-    const int nang = (g.nAng + ngroup - 1) / ngroup, waves = nch > 1 ? 16 : 8;
+    const int nang = scatter_angles(g), waves = nch > 1 ? 16 : 8;
+    // columns are split where a block's waves would get fewer than four tasks each
     const double cols = 1.3 * ST * g.s / (g.pitch_iso * (g.pixnum / g.H)) + 2.0;  // a tile's, about
     const int nsplit = (int)std::max(1.0, std::min(std::ceil(4.0 * waves / nang), std::min(cols, 1.0e6) / 3.0));
     const double rps = g.t / (g.pitch_iso * (g.pixnum / g.H));  // rows per slice

@@ -493,12 +493,24 @@ __device__ __forceinline__ double first_lane(double x) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// True when the condition holds on any lane of the wave (the host build walks one lane at a time).
+// True when the condition holds on any lane of the wave, and the least of the lanes' values.  (The host build walks one lane
+// at a time, unless it steps the lanes together itself: VCBCT_HOST_ANY_LANE and VCBCT_HOST_LANES_MIN.)
 __host__ __device__ __forceinline__ bool any_lane(bool b) {
 #ifdef __HIP_DEVICE_COMPILE__
     return __any(b);
+#elif defined(VCBCT_HOST_ANY_LANE)
+    return VCBCT_HOST_ANY_LANE(b);
 #else
     return b;
+#endif
+}
+__host__ __device__ __forceinline__ int lanes_min(int v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_readfirstlane(wave_min(v));
+#elif defined(VCBCT_HOST_LANES_MIN)
+    return VCBCT_HOST_LANES_MIN(v);
+#else
+    return v;
 #endif
 }
 

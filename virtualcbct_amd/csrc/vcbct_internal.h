@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <climits>
 #include <cstdarg>
 #include <cstdint>
 #include <string>
@@ -247,9 +249,40 @@ int launch_adjoint_multi(const ProjGeom& g, const double* tables, const void* vo
 // kernels' order, so that the rows of a wave are contiguous), and the tile scatter's workspace behind them.
 inline size_t align16(size_t n) { return (n + 15) & ~(size_t)15; }
 size_t adjoint_coef_bytes(const ProjGeom& g);
-// The scatter by voxel tiles (scatter.hip): whether it serves the geometry, its workspace, the rays' paths (with the
-// list of columns left to the ray-ordered scatter: listed[0] of them, from listed[4] on) and the scatter itself.
-bool scatter_by_tiles(const ProjGeom& g);
+// The scatter by voxel tiles (scatter.hip): a block's tile, the angles that a block takes, and whether the form serves a
+// geometry and channel count.
+constexpr int kScatterSide = 16, kScatterSlices = 32;
+// Angle groups: at least eight blocks a CU where the angles allow it, so that the last ones leave little of the chip idle.
+inline int scatter_angles(const ProjGeom& g) {
+    const long nt = (g.N + kScatterSide - 1) / kScatterSide, nzc = (g.Nz + kScatterSlices - 1) / kScatterSlices;
+    const long tiles = std::max(1L, (long)(0.785 * nt * nt)) * nzc;
+    const int ngroup = (int)std::min<long>(g.nAng, std::max(1L, (2048 + tiles - 1) / tiles));
+    return (g.nAng + ngroup - 1) / ngroup;
+}
+// Range: 15-bit voxel indices, rows and columns (the latter formed in FP32 with margins of a fiftieth), a slice chunk per
+// grid layer, and a source well outside the volume (the tile's footprint on the panel is its corners' projection).
+// At least 4e7 ray steps, as a tile costs its clearing and its final atomics whatever it gathers; and with three
+// channels or more, which go two at a time, more than one angle a block.  Backward from saved line integrals, ray-ordered
+// against tiles, over one, two, four and six channels [us]: 64x64x20 / 90 angles of 60x60 (2.1e7 steps, one angle a block)
+// 173/110, 204/185, 295/352, 416/515; 128x128x32 / 24 angles of 128x128 (5.0e7, one) 199/108, 238/195, 341/384, 479/538;
+// 256x256x64 / 4 angles of 256x256 (6.7e7, one) 277/142, 312/258, 463/478, 641/677; 512x512x256 / 1 angle of 400x400
+// (8.2e7, one) 756/570, 1324/1302, 2077/2268, 2924/3236; with two angles a block and more tiles win: 64x64x20 / 360 angles of
+// 60x60 (8.3e7, three) 411/236, 496/329, 838/661, 1257/977; 128x128x128 / 24 angles of 128x128 (5.0e7, three) 312/300,
+// 601/418, 1140/799, 1675/1174.
+// Thin slices: the walk of a tile's rays goes by blocks of steps that hold one slice plane (and columns whose blocks hold no
+// step go to the ray-ordered scatter from a list, on 512 blocks; 2048 take the same time); where a block holds fewer
+// than about two steps, three off the plane grid, the ray-ordered form is the faster throughout.  128x128 / 48 angles of
+// 128x128, two channels, ray-ordered / tiles [us]: 0.25 mm slices (2.8 steps) 1634/1395, 0.22 (2.5) 1870/1878, 0.18 (2.0)
+// 2188/2400, 0.12 (1.3) 3049/4595; 256x256 at 1 mm: 0.198 mm (2.2) 7864/7258, 0.18 (2.0) 8549/8665; 100x100 at 2.6 mm, off
+// the plane grid: 0.5 mm (4.2) 786/743, 0.3 (2.6) 1321/1416, 0.2 (1.7) 1718/2976.
+inline bool scatter_by_tiles(const ProjGeom& g, int nch) {
+    const double reach = (0.5 * g.N + 1.0) * g.s * 3.0 + std::fabs(g.x_reg) + std::fabs(g.y_reg);
+    const double zr = (0.5 * (g.Nz + 1) + 1.0) * g.t + std::fabs(g.z_reg);
+    const double steps = (0.85 * g.sad - g.lim_u) * g.t / (zr * g.s);  // of a block, about
+    return g.N < 32768 && g.H < 32768 && g.W < 32768 && (g.Nz + kScatterSlices - 1) / kScatterSlices <= 65535 &&
+           reach < g.sad && (size_t)g.nAng * g.W < (size_t)INT_MAX && (double)g.nAng * g.H * g.W * g.N >= 4.0e7 &&
+           (nch <= 2 || scatter_angles(g) > 1) && steps >= (g.aligned ? 2.2 : 3.0);
+}
 size_t scatter_work_bytes(const ProjGeom& g);
 int launch_scatter_rays(const ProjGeom& g, const double* tables, void* work, hipStream_t st, const int** listed);
 int launch_scatter_tiles(const ProjGeom& g, const double* tables, const void* work, const float* coef, int nch,
