@@ -331,6 +331,15 @@ __device__ __forceinline__ float2* fft_lds(float2* x, float2* y, const float2* T
     return x;
 }
 
+// The cosine weight 100 / sqrt(1e4 + pos1^2 + pos2^2), pos2sq = 1e4 + pos2^2: the hardware root (one ulp) and one Newton
+// step, rounded once.  Error against 64 bits over a panel: 2.8e-8 rms, 9.7e-8 at most; the root alone 4.1e-8 and 1.5e-7, a
+// square root and a division 3.4e-8 and 1.2e-7.  The filter of 360 projections of 400x400 takes 260 us with it, 258 with
+// the root alone.
+__device__ __forceinline__ float cos_weight(float pos1, float pos2sq) {
+    const float x = fmaf(pos1, pos1, pos2sq), r = __builtin_amdgcn_rsqf(x);
+    return fmaf(100.0f, r, 50.0f * r * fmaf(-(x * r), r, 1.0f));
+}
+
 // ecol (half-fan plans): the offset weighting fused into the load.  The caller's panel has Wsrc columns,
 // placed at column `off` of the W-column padded panel; a real column c of projection th contributes
 // ecol[th][c] (-log p) (= -log p^(2w), the weighted pixel's line integral; exponent 0 gives 0 whatever p), a
@@ -412,7 +421,7 @@ __global__ __launch_bounds__(FT) void k_filter(const float* __restrict__ proj, f
             const float pos2sq = fmaf(pos2, pos2, 10000.0f);
             for (int m = threadIdx.x; m < W; m += FT) {
                 float pos1 = fabsf(xc_tab[th] + (float)m) * pitchW;
-                const float cm = 100.0f * __builtin_amdgcn_rsqf(fmaf(pos1, pos1, pos2sq));
+                const float cm = cos_weight(pos1, pos2sq);
                 float v = (s == 0) ? X[m].x : X[m].y;
                 out[r * W + m] = v * cm;
             }
@@ -587,7 +596,7 @@ __global__ __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(4, 4)))
             for (int k = 0; k < 8; ++k) {
                 const int m = lane + 64 * k;
                 const float pos1 = fabsf(xc + (float)m) * pitchW;
-                const float cm = 100.0f * __builtin_amdgcn_rsqf(fmaf(pos1, pos1, pos2sq));
+                const float cm = cos_weight(pos1, pos2sq);
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, (h ? v[k].y : v[k].x) * cm), o, m * 4, 0,
                                                       0);
             }
