@@ -445,7 +445,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t bp_rsrc(const float* p, int by
 // 360 projections of 400x400: 442 us with k_filter (LDS 55 %, table loads in the vector L1 55 %, vector issue 50 % of the
 // cycles), 255 us with this kernel (vector issue 85 %).
 constexpr int FW = 4;                // waves per block
-constexpr int FWP = 4;               // row pairs per wave
 constexpr int FWS = 64 + 4;          // LDS stride of a 64-point transform (2 lanes a bank pair, the least for 8 bytes)
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
@@ -523,83 +522,81 @@ __global__ __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(4, 4)))
     const bool last = p4 == 3;
     const long r1 = 2 * ((long)blockIdx.x * FW + wave);
     if (r1 >= nrows) return;  // (uniform over the wave; the waves share nothing)
-    {
-        const bool has2 = r1 + 1 < nrows;
-        const float* p1 = proj + r1 * ws;
-        const float* p2 = has2 ? p1 + ws : p1;
-        const float* e1 = HF ? ecol + r1 / H * Wsrc : nullptr;
-        const float* e2 = HF ? ecol + (has2 ? r1 + 1 : r1) / H * Wsrc : nullptr;
-        float2 v[16];
+    const bool has2 = r1 + 1 < nrows;
+    const float* p1 = proj + r1 * ws;
+    const float* p2 = has2 ? p1 + ws : p1;
+    const float* e1 = HF ? ecol + r1 / H * Wsrc : nullptr;
+    const float* e2 = HF ? ecol + (has2 ? r1 + 1 : r1) / H * Wsrc : nullptr;
+    float2 v[16];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {  // (past the caller's columns: the nearest, not used)
-            const int c = min(max(lane + 64 * k - of, 0), ws - 1);
-            v[k] = make_float2(p1[c], p2[c]);
+    for (int k = 0; k < 8; ++k) {  // (past the caller's columns: the nearest, not used)
+        const int c = min(max(lane + 64 * k - of, 0), ws - 1);
+        v[k] = make_float2(p1[c], p2[c]);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int c = lane + 64 * k - of;
+        const bool in = c >= 0 && c < ws;  // padding: a line integral of 0
+        float a = -logf(v[k].x), b = -logf(v[k].y);
+        if (HF) {
+            const int cc = min(max(c, 0), ws - 1);
+            const float x1 = e1[cc], x2 = e2[cc];
+            a = x1 == 0.f ? 0.f : x1 * a;
+            b = x2 == 0.f ? 0.f : x2 * b;
         }
+        v[k] = make_float2(in ? a : 0.f, in && has2 ? b : 0.f);
+    }
+    dft16<false, true>(v);
+#pragma unroll
+    for (int i = 1; i < 16; ++i) v[i] = cmulc<false>(v[i], wt[(16 + i - 1) * 64 + lane]);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) S[i * FWS + lane] = v[i];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = S[q4 * FWS + p4 + 4 * i];
+    __builtin_amdgcn_wave_barrier();
+    dft16<false, false>(v);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        float2 x = i ? cmulc<false>(v[i], wt[(31 + i - 1) * 64 + lane]) : v[i];
+        // the quad's DFT over p, decimated in frequency: lanes p and p ^ 2, -i on lane 3, lanes p and p ^ 1
+        x = make_float2(fmaf(x.x, s2, quad2(x.x)), fmaf(x.y, s2, quad2(x.y)));
+        x = last ? crot<false>(x) : x;
+        x = make_float2(fmaf(x.x, s1, quad1(x.x)), fmaf(x.y, s1, quad1(x.y)));
+        x = cmulc<false>(x, wt[i * 64 + lane]);
+        // and back
+        x = make_float2(fmaf(x.x, s1, quad1(x.x)), fmaf(x.y, s1, quad1(x.y)));
+        x = last ? crot<true>(x) : x;
+        x = make_float2(fmaf(x.x, s2, quad2(x.x)), fmaf(x.y, s2, quad2(x.y)));
+        v[i] = i ? cmulc<true>(x, wt[(31 + i - 1) * 64 + lane]) : x;
+    }
+    dft16<true, false>(v);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) S[q4 * FWS + p4 + 4 * i] = v[i];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const float2 x = S[i * FWS + lane];
+        v[i] = i ? cmulc<true>(x, wt[(16 + i - 1) * 64 + lane]) : x;
+    }
+    dft16<true, false>(v);  // (k < 8 of it)
+    // cosine weight at the output pixel (F/filterSinogram.cpp:92-99, applied at :103 and :108)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (h == 1 && !has2) break;
+        const long r = r1 + h;
+        const int th = (int)(r / H), n = (int)(r % H);
+        const float pos2 = fabsf(yc_tab[th] + (float)n) * pitchW;
+        const float pos2sq = fmaf(pos2, pos2, 10000.0f), xc = xc_tab[th];
+        const __amdgpu_buffer_rsrc_t o = bp_rsrc(out + r * W, W * 4);  // (columns past the row are dropped)
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const int c = lane + 64 * k - of;
-            const bool in = c >= 0 && c < ws;  // padding: a line integral of 0
-            float a = -logf(v[k].x), b = -logf(v[k].y);
-            if (HF) {
-                const int cc = min(max(c, 0), ws - 1);
-                const float x1 = e1[cc], x2 = e2[cc];
-                a = x1 == 0.f ? 0.f : x1 * a;
-                b = x2 == 0.f ? 0.f : x2 * b;
-            }
-            v[k] = make_float2(in ? a : 0.f, in && has2 ? b : 0.f);
-        }
-        dft16<false, true>(v);
-#pragma unroll
-        for (int i = 1; i < 16; ++i) v[i] = cmulc<false>(v[i], wt[(16 + i - 1) * 64 + lane]);
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < 16; ++i) S[i * FWS + lane] = v[i];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = S[q4 * FWS + p4 + 4 * i];
-        __builtin_amdgcn_wave_barrier();
-        dft16<false, false>(v);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float2 x = i ? cmulc<false>(v[i], wt[(31 + i - 1) * 64 + lane]) : v[i];
-            // the quad's DFT over p, decimated in frequency: lanes p and p ^ 2, -i on lane 3, lanes p and p ^ 1
-            x = make_float2(fmaf(x.x, s2, quad2(x.x)), fmaf(x.y, s2, quad2(x.y)));
-            x = last ? crot<false>(x) : x;
-            x = make_float2(fmaf(x.x, s1, quad1(x.x)), fmaf(x.y, s1, quad1(x.y)));
-            x = cmulc<false>(x, wt[i * 64 + lane]);
-            // and back
-            x = make_float2(fmaf(x.x, s1, quad1(x.x)), fmaf(x.y, s1, quad1(x.y)));
-            x = last ? crot<true>(x) : x;
-            x = make_float2(fmaf(x.x, s2, quad2(x.x)), fmaf(x.y, s2, quad2(x.y)));
-            v[i] = i ? cmulc<true>(x, wt[(31 + i - 1) * 64 + lane]) : x;
-        }
-        dft16<true, false>(v);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) S[q4 * FWS + p4 + 4 * i] = v[i];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const float2 x = S[i * FWS + lane];
-            v[i] = i ? cmulc<true>(x, wt[(16 + i - 1) * 64 + lane]) : x;
-        }
-        dft16<true, false>(v);  // (k < 8 of it)
-        // cosine weight at the output pixel (F/filterSinogram.cpp:92-99, applied at :103 and :108)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (h == 1 && !has2) break;
-            const long r = r1 + h;
-            const int th = (int)(r / H), n = (int)(r % H);
-            const float pos2 = fabsf(yc_tab[th] + (float)n) * pitchW;
-            const float pos2sq = fmaf(pos2, pos2, 10000.0f), xc = xc_tab[th];
-            const __amdgpu_buffer_rsrc_t o = bp_rsrc(out + r * W, W * 4);  // (columns past the row are dropped)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int m = lane + 64 * k;
-                const float pos1 = fabsf(xc + (float)m) * pitchW;
-                const float cm = cos_weight(pos1, pos2sq);
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, (h ? v[k].y : v[k].x) * cm), o, m * 4, 0,
-                                                      0);
-            }
+            const int m = lane + 64 * k;
+            const float pos1 = fabsf(xc + (float)m) * pitchW;
+            const float cm = cos_weight(pos1, pos2sq);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, (h ? v[k].y : v[k].x) * cm), o, m * 4, 0,
+                                                  0);
         }
     }
 }
