@@ -429,23 +429,28 @@ struct OrderedAcc : RunAcc<VoxT> {
     using RunAcc<VoxT>::kBatch;
     static constexpr bool kSecondFirst = !std::is_same<VoxT, float4>::value;
     __device__ __forceinline__ OrderedAcc(const VoxT* vox, const ProjGeom& g) : RunAcc<VoxT>(vox, g) {}
+    // Pieces [i, i + B) of the list, those past pb with length 0 off the volume.
+    template <int B>
+    __device__ __forceinline__ void batch_ordered(const OrderedPiece* p, int i, int pb, int px, int first_new, float lo,
+                                                  int zo, int zn, double K) {
+        OrderedPiece t[B];
+        Q q[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) t[b] = p[i + b < pb ? i + b : pb - 1];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int z = i + b < first_new || i + b == px ? zo : zn;
+            this->load(t[b].cb + (i + b < pb ? z : RunAcc<VoxT>::kOut), q[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+            this->add(q[b], i + b >= pb ? 0.0f : i + b == px ? lo : (float)(t[b].len * K));
+    }
     __device__ __forceinline__ void run_ordered(const OrderedPiece* p, int pa, int pb, int px, int first_new, float lo,
                                                 int zo, int zn, double K) {
-        for (int i = pa; i < pb; i += kBatch) {
-            OrderedPiece t[kBatch];
-            Q q[kBatch];
-            // (past the end: the last piece's column with length 0, off the volume)
-#pragma unroll
-            for (int b = 0; b < kBatch; ++b) t[b] = p[i + b < pb ? i + b : pb - 1];
-#pragma unroll
-            for (int b = 0; b < kBatch; ++b) {
-                const int z = i + b < first_new || i + b == px ? zo : zn;
-                this->load(t[b].cb + (i + b < pb ? z : RunAcc<VoxT>::kOut), q[b]);
-            }
-#pragma unroll
-            for (int b = 0; b < kBatch; ++b)
-                this->add(q[b], i + b >= pb ? 0.0f : i + b == px ? lo : (float)(t[b].len * K));
-        }
+        int i = pa;
+        for (; i + kBatch <= pb; i += kBatch) batch_ordered<kBatch>(p, i, i + kBatch, px, first_new, lo, zo, zn, K);
+        if (i < pb) batch_ordered<kBatch - 1>(p, i, pb, px, first_new, lo, zo, zn, K);
     }
 };
 
