@@ -34,10 +34,13 @@ namespace vcbct {
 #define VCBCT_WAVES8 __attribute__((amdgpu_waves_per_eu(8, 8)))
 // The projection kernels that hold the step walk alone (volumes past the run walk's reach, thin slices, segment counts)
 // are held to 7, the intensity to 8: 700x700x600 two-channel slices / 12 angles of 400x400, log projection 3.9 ms at 5
-// waves, 3.7 at 7.
+// waves, 3.7 at 7.  Those that walk by runs hold the run walk of one kind of plane grid: with both in one kernel six to
+// fifteen registers were spilled (the full scan 10.66 ms against 10.45, 640x640 u16 maps 1.47 against 1.40).
+enum { WALK_STEPS = 0, WALK_ANY = 1, WALK_ALIGNED = 2, WALK_OFF = 3 };  // the walks that a kernel holds: run walks on / off the plane grid
 #define VCBCT_WAVES_RUN __attribute__((amdgpu_waves_per_eu(5, 5)))
-#define VCBCT_WAVES_FWD(MODE, RUNS)               \
-    __attribute__((amdgpu_waves_per_eu((RUNS) ? 5 : (MODE) == VCBCT_MODE_INTENSITY ? 8 : 7, (RUNS) ? 5 : 8)))
+#define VCBCT_WAVES_FWD(MODE, WALK)                                                                          \
+    __attribute__((amdgpu_waves_per_eu((WALK) != WALK_STEPS ? 5 : (MODE) == VCBCT_MODE_INTENSITY ? 8 : 7, \
+                                       (WALK) != WALK_STEPS ? 5 : 8)))
 #define VCBCT_WAVES_COEF(MODE, RUNS)                                                                   \
     __attribute__((amdgpu_waves_per_eu(!(RUNS) ? 8 : (MODE) == VCBCT_ADJ_LOSS ? 4 : 5,                  \
                                        !(RUNS) ? 8 : (MODE) == VCBCT_ADJ_LOSS ? 4 : 5)))
@@ -471,9 +474,8 @@ __host__ __device__ __forceinline__ bool run_walk(const ProjGeom& g) {
 
 // The line integrals of one wave's rays into L: by runs where the wave's lanes share their xy path, a block holds enough
 // steps (two slice planes in one step: none) and the volume is within the gathers' reach, else step by step.
-// ORDERED: bit for bit the step walk's sums (plane grids off the voxel grid keep that walk).  RUNS false: the step walk
-// alone (run_walk).  Returns the lane's cos^3 factor.
-template <bool ORDERED, bool RUNS, class VoxT>
+// ORDERED: bit for bit the step walk's sums (plane grids off the voxel grid keep that walk).  Returns the lane's cos^3 factor.
+template <bool ORDERED, int WALK, class VoxT>
 __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double sn, double xc, double yc, int j, int jj,
                                            bool active, const VoxT* __restrict__ vox, float (&L)[VCBCT_MAX_MAT],
                                            WalkLds* lds) {
@@ -497,7 +499,7 @@ __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double s
     if (kmin > kmax) return r.leng;  // no lane reaches the volume's z band
     const bool same = __all((int)r.swap == __builtin_amdgcn_readfirstlane((int)r.swap));
     int nb = 0;
-    if constexpr (RUNS) {
+    if constexpr (WALK != WALK_STEPS) {
         // (the ordered walk hands pieces over when any lane crosses a slice, in range or not)
         float slope = (ORDERED ? active && r.hit : klo <= khi) ? run_slope(r) : 0.0f;
 #pragma unroll
@@ -505,7 +507,7 @@ __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double s
         if (same && run_walk<VoxT>(g)) nb = __builtin_amdgcn_readfirstlane(run_block_steps(g, slope));
         if (nb < kRunSteps<ORDERED> || (ORDERED && !g.aligned)) nb = 0;
     }
-    if (RUNS && nb > 0) {
+    if (WALK != WALK_STEPS && nb > 0) {
         if constexpr (ORDERED) {
             OrderedAcc<VoxT> acc(vox, g);
             walk_runs_ordered(g, r, active, kmin, kmax, nb, acc, &lds->ordered);
@@ -513,7 +515,7 @@ __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double s
             for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
         } else {
             RunAcc<VoxT> acc(vox, g);
-            if (g.aligned) walk_runs<true>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
+            if (WALK == WALK_ALIGNED || (WALK == WALK_ANY && g.aligned)) walk_runs<true>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
             else walk_runs<false>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
 #pragma unroll
             for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
@@ -742,7 +744,7 @@ bool tile_shape_valid(const TileShape& s) {
 }
 
 // One wave: 64 detector rows [64 rg, 64 rg + 64) of column jj at angle a.  Wave-uniform arguments.
-template <int MODE, class VoxT, bool RUNS>
+template <int MODE, class VoxT, int WALK>
 __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __restrict__ tab,
                                              const VoxT* __restrict__ vox, const double* __restrict__ mu,
                                              const double* __restrict__ pdf, const float* __restrict__ muf,
@@ -764,7 +766,7 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
         return;
     }
     float L[VCBCT_MAX_MAT];
-    const double leng = sum_wave<false, RUNS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
+    const double leng = sum_wave<false, WALK>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
     if (!active) return;
 
     if (MODE == VCBCT_MODE_LINEINT) {
@@ -826,8 +828,8 @@ __device__ __forceinline__ void forward_wave(const ProjGeom& g, const double* __
 }
 
 // WPB waves per block (TileShape: rgb * cols); the block's waves share nothing but the LDS allocation.
-template <int MODE, class VoxT, int WPB, bool RUNS>
-__global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_FWD(MODE, RUNS) void k_forward(ProjGeom g, const double* __restrict__ tab,
+template <int MODE, class VoxT, int WPB, int WALK>
+__global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_FWD(MODE, WALK) void k_forward(ProjGeom g, const double* __restrict__ tab,
                                                                  const VoxT* __restrict__ vox,
                                                                  const double* __restrict__ mu,
                                                                  const double* __restrict__ pdf,
@@ -838,7 +840,7 @@ __global__ __launch_bounds__(64 * WPB) VCBCT_WAVES_FWD(MODE, RUNS) void k_forwar
     __shared__ WalkLds steps[WPB];
     const Tile t = tile_map(tm, nA);
     if (t.col >= g.W || t.a >= nA || t.rg * 64 >= g.H) return;  // wave out of range: uniform exit
-    forward_wave<MODE, VoxT, RUNS>(g, tab, vox, mu, pdf, muf, pdff, NE, inv_xf, nl, a0 + t.a, t.rg, t.col, out, aux,
+    forward_wave<MODE, VoxT, WALK>(g, tab, vox, mu, pdf, muf, pdff, NE, inv_xf, nl, a0 + t.a, t.rg, t.col, out, aux,
                              &steps[threadIdx.x >> 6]);
 }
 
@@ -884,7 +886,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_RUN void k_forward_batch(const Bat
             const int a = P.split ? q * P.pang + al : al;
             const int jj = P.split ? cl : q * P.pcols + cl;
             if (jj >= P.g.W || a >= P.g.nAng) continue;
-            forward_wave<VCBCT_MODE_INTENSITY, VoxT, true>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
+            forward_wave<VCBCT_MODE_INTENSITY, VoxT, WALK_ANY>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
                                                      P.inv_xf, P.g.nmat, a, rg, jj, P.out, nullptr,
                                                      &steps[threadIdx.x >> 6]);
         }
@@ -907,7 +909,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_RUN void k_forward_flat(const Batc
     const BatchProblem& P = pr[lo];
     const Tile t = tile_map(P.tm, P.g.nAng, b - P.block_start);
     if (t.col >= P.g.W || t.a >= P.g.nAng || t.rg * 64 >= P.g.H) return;  // wave out of range: uniform exit
-    forward_wave<VCBCT_MODE_INTENSITY, VoxT, true>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
+    forward_wave<VCBCT_MODE_INTENSITY, VoxT, WALK_ANY>(P.g, P.tab, (const VoxT*)P.vox, P.mu, P.pdf, P.muf, P.pdff, P.NE,
                                              P.inv_xf, P.g.nmat, t.a, t.rg, t.col, P.out, nullptr,
                                              &steps[threadIdx.x >> 6]);
 }
@@ -1028,7 +1030,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_COEF(MODE, RUNS) void k_adjoint_co
     const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
                  yc = ldk(tab, 3 * g.nAng + a);
     float L[VCBCT_MAX_MAT];
-    sum_wave<MODE == VCBCT_ADJ_LOSS, RUNS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
+    sum_wave<MODE == VCBCT_ADJ_LOSS, RUNS ? WALK_ANY : WALK_STEPS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
 
     double lossc = 0.0;
     if (active) {
@@ -1111,7 +1113,7 @@ __global__ __launch_bounds__(256) VCBCT_WAVES_MULTI(RUNS) void k_adjoint_coef_mu
     const double c = ldk(tab, a), sn = ldk(tab, g.nAng + a), xc = ldk(tab, 2 * g.nAng + a),
                  yc = ldk(tab, 3 * g.nAng + a);
     float L[VCBCT_MAX_MAT];
-    sum_wave<true, RUNS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
+    sum_wave<true, RUNS ? WALK_ANY : WALK_STEPS>(g, c, sn, xc, yc, j, jj, active, vox, L, steps);
 
     double lossc = 0.0;
     if (active) {
@@ -1345,24 +1347,25 @@ template <int M, class T>
 static void launch_fwd_t(int wpb, dim3 grid, hipStream_t st, const ProjGeom& g, const double* tables, const void* vox,
                          const Spectrum& sp, double inv_xf, int a0, int nA, const TileMap& tm, float* out,
                          float* aux) {
-#define VCBCT_LAUNCH_FWD(W, RUNS)                                                                             \
-    hipLaunchKernelGGL((k_forward<M, T, W, RUNS>), grid, dim3(64 * W), 0, st, g, tables, (const T*)vox, sp.mu, sp.pdf, \
+#define VCBCT_LAUNCH_FWD(W, WALK)                                                                             \
+    hipLaunchKernelGGL((k_forward<M, T, W, WALK>), grid, dim3(64 * W), 0, st, g, tables, (const T*)vox, sp.mu, sp.pdf, \
                        sp.muf, sp.pdff, sp.NE, inv_xf, sp.nl, a0, nA, tm, out, aux)
+#define VCBCT_LAUNCH_FWD_W(WALK)                    \
+    do {                                            \
+        if (wpb == 2) VCBCT_LAUNCH_FWD(2, WALK);      \
+        else if (wpb == 8) VCBCT_LAUNCH_FWD(8, WALK); \
+        else VCBCT_LAUNCH_FWD(4, WALK);             \
+    } while (0)
     if constexpr (M == VCBCT_MODE_INTENSITY || M == VCBCT_MODE_LOGPROJ) {
-        if (run_walk<T>(g)) {
-            if (wpb == 2) VCBCT_LAUNCH_FWD(2, true);
-            else if (wpb == 8) VCBCT_LAUNCH_FWD(8, true);
-            else VCBCT_LAUNCH_FWD(4, true);
-        } else {
-            if (wpb == 2) VCBCT_LAUNCH_FWD(2, false);
-            else if (wpb == 8) VCBCT_LAUNCH_FWD(8, false);
-            else VCBCT_LAUNCH_FWD(4, false);
-        }
+        if (!run_walk<T>(g)) VCBCT_LAUNCH_FWD_W(WALK_STEPS);
+        else if (g.aligned) VCBCT_LAUNCH_FWD_W(WALK_ALIGNED);
+        else VCBCT_LAUNCH_FWD_W(WALK_OFF);
     } else if constexpr (M == VCBCT_MODE_LINEINT) {
-        VCBCT_LAUNCH_FWD(4, true);
+        VCBCT_LAUNCH_FWD(4, WALK_ANY);
     } else {
-        VCBCT_LAUNCH_FWD(4, false);
+        VCBCT_LAUNCH_FWD(4, WALK_STEPS);
     }
+#undef VCBCT_LAUNCH_FWD_W
 #undef VCBCT_LAUNCH_FWD
 }
 

@@ -281,7 +281,7 @@ inline bool scatter_by_tiles(const ProjGeom& g, int nch) {
     const double steps = (0.85 * g.sad - g.lim_u) * g.t / (zr * g.s);  // of a block, about
     return g.N < 32768 && g.H < 32768 && g.W < 32768 && (g.Nz + kScatterSlices - 1) / kScatterSlices <= 65535 &&
            reach < g.sad && (size_t)g.nAng * g.W < (size_t)INT_MAX && (double)g.nAng * g.H * g.W * g.N >= 4.0e7 &&
-           (nch <= 2 || scatter_angles(g) > 1) && steps >= (g.aligned ? 2.2 : 3.0);
+           (nch <= 2 || scatter_angles(g) > 1) && steps >= (g.aligned ? 2.3 : 3.0);
 }
 size_t scatter_work_bytes(const ProjGeom& g);
 int launch_scatter_rays(const ProjGeom& g, const double* tables, void* work, hipStream_t st, const int** listed);
