@@ -165,7 +165,7 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
 #else
     const RayCtx& r = r_in;
 #endif
-    constexpr bool kEarly = sizeof(typename Acc::Q) <= 8;
+    constexpr bool kEarly = sizeof(typename Acc::Q) <= (ALIGNED ? 8 : 12);
     const bool on = active && r.hit;
     const ChargeC c = charge_consts(g, r);
     const double u0 = r.uin;
@@ -291,10 +291,11 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
                         c2 = l2 > 0.0f ? cb + zn : (int)Acc::kOut;
                     }
                 }
-                // The parts' gathers go out before the block's and are added after it (kEarly, two-channel records): waiting
-                // for them here, or after the main loop, costs the wave a memory latency each per block (320x320x77 at
-                // 0.977 mm / 120 angles: 2.02 ms against 1.86).  Larger records would spill for it (u16 maps: 1.46 against
-                // 1.43 ms), so theirs are gathered after it; the order of the sums is the same.
+                // The parts' gathers go out before the block's and are added after it (kEarly): waiting for them here, or after
+                // the main loop, costs the wave a memory latency each per block (320x320x77 at 0.977 mm / 120 angles over
+                // two channels 2.02 ms against 1.86; 458x458x21 at 0.598 mm / 120 angles over u16 maps 624 against
+                // 590 us).  Records for which that takes registers from the gathers themselves are gathered after it
+                // (u16 maps on the plane grid: 1.40 against 1.42 ms); the order of the sums is the same.
                 if (any_lane(special)) {
                     // the parts from their own midpoints, off the list; with equal crossing distances the whole chord
                     // once, in place of both pieces
