@@ -28,15 +28,17 @@ namespace vcbct {
 // Occupancy of the ray kernels.  The scatter walks step by step and waits on dependent LDS reads and scalar
 // broadcasts; more resident waves hide that better than spilling a few registers costs: held to 8 waves per SIMD.
 // The kernels that walk by runs (runs.h) keep eight gathers of a wave in flight instead, for which 5 waves per
-// SIMD have the registers: the 512x512x128 / 360-angle projection takes 10.7 ms at 5 waves, 10.9 at 6, 11.5 at 7
-// and 12.6 at 8 (where the scalar registers spill too); with the step walk it took 20.7 ms.  The ordered form needs
-// 4 (54.1 ms for the dual-energy gradient of a 512x512x64 / 360-angle problem; 54.6 at 5 with spills).
+// SIMD have the registers: the 512x512x128 / 360-angle projection takes 10.45 ms at 5 waves (10.51 at 4; with both run
+// walks in one kernel 10.7 at 5, 10.9 at 6, 11.5 at 7 and 12.6 at 8, where the scalar registers spill too); with the step
+// walk it took 20.7 ms.  The ordered form needs 4 (27.9 ms for the dual-energy gradient of a 512x512x64 / 360-angle
+// problem; 28.2 at 5 with spills).
 #define VCBCT_WAVES8 __attribute__((amdgpu_waves_per_eu(8, 8)))
 // The projection kernels that hold the step walk alone (volumes past the run walk's reach, thin slices, segment counts)
 // are held to 7, the intensity to 8: 700x700x600 two-channel slices / 12 angles of 400x400, log projection 3.9 ms at 5
 // waves, 3.7 at 7.  Those that walk by runs hold the run walk of one kind of plane grid: with both in one kernel six to
 // fifteen registers were spilled (the full scan 10.66 ms against 10.45, 640x640 u16 maps 1.47 against 1.40).
-enum { WALK_STEPS = 0, WALK_ANY = 1, WALK_ALIGNED = 2, WALK_OFF = 3 };  // the walks that a kernel holds: run walks on / off the plane grid
+// The walks that a kernel holds: ALIGNED / OFF the run walk on / off the plane grid.
+enum { WALK_STEPS = 0, WALK_ANY = 1, WALK_ALIGNED = 2, WALK_OFF = 3 };
 #define VCBCT_WAVES_RUN __attribute__((amdgpu_waves_per_eu(5, 5)))
 #define VCBCT_WAVES_FWD(MODE, WALK)                                                                          \
     __attribute__((amdgpu_waves_per_eu((WALK) != WALK_STEPS ? 5 : (MODE) == VCBCT_MODE_INTENSITY ? 8 : 7, \
@@ -515,8 +517,10 @@ __device__ __forceinline__ double sum_wave(const ProjGeom& g, double c, double s
             for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
         } else {
             RunAcc<VoxT> acc(vox, g);
-            if (WALK == WALK_ALIGNED || (WALK == WALK_ANY && g.aligned)) walk_runs<true>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
-            else walk_runs<false>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
+            if (WALK == WALK_ALIGNED || (WALK == WALK_ANY && g.aligned))
+                walk_runs<true>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
+            else
+                walk_runs<false>(g, r, active, kmin, kmax, nb, acc, &lds->runs);
 #pragma unroll
             for (int m = 0; m < VCBCT_MAX_MAT; ++m) L[m] = acc.L[m];
         }

@@ -18,12 +18,13 @@
 // the midpoint, and equal crossing distances charge the whole chord once.  Where those need a part's own midpoint
 // (a step at the circle's boundary, equal distances, a plane grid off the voxel grid) the parts are formed as the
 // step walk forms its segments.
-// What bounds it: on the 512x512x128 / 360-angle projection the gathers' traffic beyond L2 (7.7e10 bytes at 7.4 TB/s);
-// the step walk took 20.7 ms there, bound by vector issue (1.19e10 wave-instructions, now 4.5e9), this walk 10.5 ms.
+// What bounds it: on the 512x512x128 / 360-angle projection the gathers' traffic beyond L2 (7.6e10 bytes at 7.3 TB/s);
+// the step walk took 20.7 ms there, bound by vector issue (1.19e10 wave-instructions, now 4.6e9), this walk 10.45 ms.
 // A piece's length is its extent along the major axis times the ray's length factor, formed in FP64 and rounded once per
-// piece as the step walk does (extent and factor rounded to FP32 first shift a whole ray by up to 6e-8; the full scan takes
-// the same 10.7 ms, 320x320x77 at 0.977 mm / 120 angles 1.87 against 1.80 ms, six u16 maps 1.47 against 1.50): FP32 sums of equal terms (a constant map) round one way, and by the terms' own digits, so lengths scaled
-// once at the end would leave a log projection 1e-7 off the step walk's there.
+// piece as the step walk does.  Extent and factor rounded to FP32 first would shift a whole ray by up to 6e-8; the full scan
+// takes the same time either way, 320x320x77 at 0.977 mm / 120 angles 1.87 against 1.80 ms, six u16 maps 1.47 against
+// 1.50.  FP32 sums of equal terms (a constant map) round one way, and by the terms' own digits, so lengths scaled once at
+// the end would leave a log projection 1e-7 off the step walk's there.
 #pragma once
 
 #include "traverse.h"
@@ -346,12 +347,13 @@ __host__ __device__ __forceinline__ void walk_runs(const ProjGeom& g, const RayC
 }
 
 // The run walk in the step walk's order of additions, for sums that must come out bit for bit as the step walk's
-// (traverse_table, aligned plane grids): the log projection and the losses formed from it, whose FP64 sums would
-// otherwise move by ~1e-6 where a fit holds constant maps (FP32 sums of equal terms round one way).  A piece's length
-// is rounded as (float)(|b - a| K) per ray; a split step adds its second piece before its first where
-// the step walk's pipelined gather does (Acc::kSecondFirst); a crossing lane's first part is charged in its place and the second held and handed
-// over where the step walk hands it over (before the step in which a lane that holds a piece crosses again).  Steps at
-// the circle's boundary, and the rare ones with equal crossing distances, run as the step walk runs them.
+// (traverse_table, aligned plane grids): the loss forms of the coefficient kernels, whose FP64 losses would otherwise move
+// by ~1e-6 where a fit holds constant maps (FP32 sums of equal terms round one way).  The log projection takes walk_runs,
+// so a loss formed from it differs from the fused one by that much.  A piece's length is rounded as (float)(|b - a| K) per
+// ray; a split step adds its second piece before its first where the step walk's pipelined gather does
+// (Acc::kSecondFirst); a crossing lane's first part is charged in its place and the second held and handed over where the
+// step walk hands it over (before the step in which a lane that holds a piece crosses again).  Steps at the circle's
+// boundary, and the rare ones with equal crossing distances, run as the step walk runs them.
 // Ten vector instructions per piece and channel pair.
 template <class Acc>
 __host__ __device__ __forceinline__ void walk_runs_ordered(const ProjGeom& g, const RayCtx& r_in, bool active,

@@ -6,9 +6,9 @@
 // dual-energy gradient of a 512x512x64 / 360-angle problem.  Here a block owns a tile of ST x ST voxel columns by SZ
 // slices in LDS, visits every ray that crosses the tile at the angles of its group, and adds the tile to the gradient
 // once at the end, so that a voxel costs one global atomic per angle group instead of one per ray.
-// Measured: that scatter 38.8 -> 13.1 ms, 256x256x64 / 360 angles / one channel 11.4 -> 6.0 ms, 256x256x64 / 90 angles of
-// 256x256 / two channels 2.87 -> 1.2 ms.  What bounds it now is vector issue (4.8e9 wave-instructions, 60 % of the
-// cycles; a fifth of them the steps of the columns, formed anew for every tile) beside the LDS atomics (55 %).
+// Measured: that scatter 38.8 -> 13.15 ms, 256x256x64 / 360 angles / one channel 11.4 -> 6.1 ms, 256x256x64 / 90 angles of
+// 256x256 / two channels 2.87 -> 1.2 ms.  What bounds it now is vector issue (5.0e9 wave-instructions, 61 % of the
+// cycles; a fifth of them the steps of the columns, formed anew for every tile) beside the LDS atomics (51 %).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
