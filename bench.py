@@ -735,7 +735,7 @@ def main():
                 "frac": achieved / HBM_PEAK_GBS, "traffic": read_traffic(),
                 "traffic_source": "profiles/forward_c2_traffic.txt: rocprofv3 FETCH_SIZE and WRITE_SIZE of this "
                                   "kernel, scaled by their readings for a plain 1 GiB copy (not measured in this run)",
-                "kernel": f"k_forward<0, {rec}, {P.tile[0] * P.tile[1]}>", "segments_per_launch": segs,
+                "kernel": f"k_forward<0, {rec}, {P.tile[0] * P.tile[1]}, 2>", "segments_per_launch": segs,
                 "algorithmic_bytes_per_launch": alg_bytes,
                 "algorithmic_bytes_note": "12 B per charged segment (six u16 maps) + 4 B per ray, the traversal's "
                                           "definition; the kernel gathers the volume's spectral channels instead",
